@@ -57,10 +57,41 @@ __device__ __forceinline__ int64_t wave_event() {
 }
 
 // ------------------------------------------------------------------ kernels
+// Minimum of each event's column of a caller's grid f (nf, n_ev), into the
+// event's record at REC_F0 (a site slot that records with a caller's grid,
+// one site at most, leave unused).  Bound by the read of f; a block takes eb
+// neighbouring events (the columns' rows are then read in runs of eb doubles)
+// and 1024 / eb lanes per event, four loads in flight per lane.  As the
+// setup's own loop, one dependent load per point and event: 507 us of setup
+// at 500 events x 2000 points, with this kernel 30 + 5 us.
+constexpr int REC_F0 = REC_SITE + (GWF_MAX_DETECTORS - 1) * SC_COUNT;
+__global__ __launch_bounds__(1024) void k_grid_min(const double* __restrict__ f, int64_t n_ev, int64_t nf, int eb,
+                                                   double* __restrict__ rec) {
+  __shared__ double red[1024];
+  const int tx = threadIdx.x % eb, ty = threadIdx.x / eb, nl = 1024 / eb;  // eb: a power of two
+  const int64_t e = (int64_t)blockIdx.x * eb + tx;
+  double m = __builtin_nan("");  // fmin drops a NaN operand
+  if (e < n_ev) {
+    const double* fe = f + e;
+    int64_t i = ty;
+    for (; i + 3 * nl < nf; i += 4 * nl) {
+      const double a = fe[i * n_ev], b = fe[(i + nl) * n_ev], c = fe[(i + 2 * nl) * n_ev], d = fe[(i + 3 * nl) * n_ev];
+      m = fmin(fmin(m, fmin(a, b)), fmin(c, d));
+    }
+    for (; i < nf; i += nl) m = fmin(m, fe[i * n_ev]);
+  }
+  red[threadIdx.x] = m;
+  __syncthreads();
+  for (int s = nl / 2; s > 0; s >>= 1) {
+    if (ty < s) red[threadIdx.x] = fmin(red[threadIdx.x], red[threadIdx.x + s * eb]);
+    __syncthreads();
+  }
+  if (ty == 0 && e < n_ev) rec[e * (int64_t)REC_DOUBLES + REC_F0] = red[tx];
+}
+
 template <int MODEL, int NT>
 __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const double* __restrict__ par, int64_t ld,
-                                               int64_t n_ev, const double* __restrict__ fgrid, int64_t nf,
-                                               double* __restrict__ rec) {
+                                               int64_t n_ev, bool own_grid, double* __restrict__ rec) {
   // IMRPhenomD models: NT lanes per event, lane tk evaluating tangent tk
   // (setup_waveform_split); TaylorF2: one lane per event
   constexpr int LPE = is_pd(MODEL) ? NT : 1;
@@ -69,9 +100,8 @@ __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const d
   const int tk = (int)(tid - e * LPE);
   if (e >= n_ev) return;
   double f0;
-  if (fgrid) {  // minimum of the caller's grid column (waveforms.py:1139)
-    f0 = fgrid[e];
-    for (int64_t i = 1; i < nf; ++i) f0 = fmin(f0, fgrid[i * n_ev + e]);
+  if (own_grid) {  // minimum of the caller's grid column (waveforms.py:1139), from k_grid_min
+    f0 = rec[e * (int64_t)REC_DOUBLES + REC_F0];
   } else {  // first grid point: 10**log10(fmin) for geomspace, fmin for linspace
     f0 = net.lin ? net.fmin : grid_f(log10(net.fmin), log10(net.fmin), 0, 1);
   }
@@ -2376,19 +2406,30 @@ int launch_setup(const gwf_waveform* wf, const NetK& net, const double* par, int
   const int64_t nt = n_ev * lpe;
   const int bs = nt <= 65536 * 4 ? 64 : 256;
   const dim3 grid((unsigned)((nt + bs - 1) / bs)), block(bs);
+  // the grid minimum is the reference frequency of the models that have none set
+  const bool own_grid = fgrid && (is_pd(wf->model) ? !(wf->fref > 0.0) : (wf->is_eccentric && !(wf->fref_ecc > 0.0)));
+  if (own_grid) {
+    const int eb = n_ev >= 16 ? 16 : (n_ev >= 4 ? 4 : 1);
+    hipLaunchKernelGGL(k_grid_min, dim3((unsigned)((n_ev + eb - 1) / eb)), dim3(1024), 0, st, fgrid, n_ev, nf, eb, rec);
+  }
   if (wf->model == GWF_MODEL_IMRPHENOMD)
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_IMRPHENOMD, 4>), grid, block, 0, st, *wf, net, par, ld, n_ev, fgrid, nf, rec);
+    hipLaunchKernelGGL((k_setup<GWF_MODEL_IMRPHENOMD, 4>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
+                       rec);
   else if (wf->model == GWF_MODEL_IMRPHENOMD_NRTIDALV2)
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_IMRPHENOMD_NRTIDALV2, 6>), grid, block, 0, st, *wf, net, par, ld, n_ev, fgrid,
-                       nf, rec);
+    hipLaunchKernelGGL((k_setup<GWF_MODEL_IMRPHENOMD_NRTIDALV2, 6>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
+                       rec);
   else if (nt_of(wf) == 5)
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 5>), grid, block, 0, st, *wf, net, par, ld, n_ev, fgrid, nf, rec);
+    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 5>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
+                       rec);
   else if (nt_of(wf) == 7)  // tidal and eccentric TaylorF2, 14 parameters
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 7>), grid, block, 0, st, *wf, net, par, ld, n_ev, fgrid, nf, rec);
+    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 7>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
+                       rec);
   else if (nt_of(wf) == 6)
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 6>), grid, block, 0, st, *wf, net, par, ld, n_ev, fgrid, nf, rec);
+    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 6>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
+                       rec);
   else
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 4>), grid, block, 0, st, *wf, net, par, ld, n_ev, fgrid, nf, rec);
+    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 4>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
+                       rec);
   return hip_check(hipGetLastError(), "setup launch");
 }
 
