@@ -195,60 +195,131 @@ __device__ __forceinline__ void pq_fail(unsigned int* counter, int lane) {
   if (lane == 0) atomicOr(counter + 1, 1u);
 }
 
-// Gram on the matrix cores: the arm rows of the chunk's 64 points, scaled by
-// sqrt(w) (w = trapezoid weight x arm weight / S), go through a per-wave LDS
-// tile X[point][param] (row stride PQ_XS doubles) and G += X^T X runs as 16
-// v_mfma_f64_16x16x4f64 per (arm, re|im): lane l feeds X[4 s + l / 16][l % 16]
-// as both operands (A[i][k] is lane i + 16 k, B[k][j] lane j + 16 k), and the
-// 16 x 16 accumulator holds G[i][j] in lane j + 16 (i % 4), element i / 4.
-// Points past res contribute zero rows; NACC accumulators rotate so that
-// consecutive MFMAs do not wait for each other.
+// Contractions over a chunk's 64 points on the matrix cores, in 4 x 4 blocks:
+// v_mfma_f64_4x4x4_4b multiplies four independent 4 x 4 (k = 4) blocks, lane
+// l holding A(row l % 4, k l / 16) and B(k l / 16, column l % 4) of block
+// (l / 4) % 4 and D(row l / 16, column l % 4) of that block.  All four blocks
+// are given the same pair of 4-column groups and different points (point
+// l / 4 of each 16), so a register read per group and 16 points feeds every
+// pair of groups it is in, and an accumulator per pair is summed over its
+// blocks at the end.  FP64 MFMA and FP64 VALU instructions run on the same
+// units (measured: a wave of each on one SIMD takes the sum of their times),
+// at the same rate in 4 x 4 x 4 and 16 x 16 x 4 form (70.5 and 77.6 TFLOP/s),
+// so every padded product costs: an 11-row Gram needs 6 block pairs (384
+// cycles per 64 points and part) where one 16 x 16 tile takes 1024, and 9
+// factors x 4 sky sums 3 (192).
+// The chunk's values go through a per-wave LDS tile X[point][column], rows
+// of G groups padded to a pitch whose 16-byte row writes and 4-column reads
+// spread over all banks (12 or 20 doubles).
 typedef double v4d __attribute__((ext_vector_type(4)));
-constexpr int PQ_XS = 17;
+constexpr int pq_pitch(int groups) { return groups <= 3 ? 12 : 20; }
+constexpr int PQ_TILE = 64 * 20;
+
+__device__ __forceinline__ double mfma_4b(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+// this lane's base in the tile for reads of (point l / 4 of 16, column l % 4)
+template <int XS>
+__device__ __forceinline__ const double* tile_at(const double* X, int lane) {
+  return X + (lane >> 2) * XS + (lane & 3);
+}
+// the sum of an accumulator over its four blocks, in every lane of (i, j)
+__device__ __forceinline__ double block_sum(double v) {
+  v += __shfl_xor(v, 4, 64);
+  return v + __shfl_xor(v, 8, 64);
+}
+
+// Gram of the arm rows (scaled by sqrt of trapezoid weight x arm weight / S),
+// bound by the FP64 units it shares with the rows' arithmetic (per-arm
+// matrices of 3001 IMRPhenomD events x 1000 points, five arms: 550 us with
+// 16 x 16 tiles, 433 us in 4 x 4 blocks):
+// acc += X^T X, real and imaginary parts.  Points past res contribute zero
+// rows; padding columns are zero.  Up to 12 rows: an accumulator per block
+// pair g <= h.  13 to 16 rows: one 16 x 16 tile, v_mfma_f64_16x16x4 with
+// X[4 t + l / 16][l % 16] as both operands and element (i, j) in lane
+// j + 16 (i % 4), item i / 4 (four doubles per arm).  The ten pairs in 4 x 4
+// blocks would take 640 instead of 1024 MFMA cycles a part but measured no
+// faster: with an accumulator per pair eight arms' sets spill (132-160
+// VGPRs), and with two pairs per instruction the operands need 40 reads of
+// the tile instead of 16 (599 us against 605 us per 3001 NRTidalv2 events x
+// 1000 points, five arms) or register moves that do not overlap an FP64 MFMA
+// (668 us).
+template <int P>
+struct GramBlocks {
+  static constexpr int G = (P + 3) / 4, XS = pq_pitch(G);
+  static constexpr int ACCS = G <= 3 ? G * (G + 1) / 2 : 4;
+};
+template <int P>
+__device__ __forceinline__ void mfma_rows(const double* re, const double* im, double* X, int lane, double* acc) {
+  typedef GramBlocks<P> B;
+  const double* rd = tile_at<B::XS>(X, lane);
+  double2* row = (double2*)(X + lane * B::XS);
+#pragma unroll
+  for (int part = 0; part < 2; ++part) {
+    const double* v = part ? im : re;
+#pragma unroll
+    for (int i = 0; i + 1 < P; i += 2) row[i / 2] = make_double2(v[i], v[i + 1]);
+    if (P & 1) row[P / 2] = make_double2(v[P - 1], 0.0);
+    __builtin_amdgcn_wave_barrier();
+    // operands read one step ahead of the products: an LDS read takes longer
+    // than a step's MFMAs
+    if constexpr (B::G == 4) {
+      const double* r4 = X + (lane >> 4) * B::XS + (lane & 15);
+      v4d c = {acc[0], acc[1], acc[2], acc[3]};
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        const double x = r4[4 * t * B::XS];
+        c = __builtin_amdgcn_mfma_f64_16x16x4f64(x, x, c, 0, 0, 0);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] = c[q];
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
+    double nx[B::G];
+#pragma unroll
+    for (int g = 0; g < B::G; ++g) nx[g] = rd[4 * g];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      double x[B::G];
+#pragma unroll
+      for (int g = 0; g < B::G; ++g) x[g] = nx[g];
+      if (t < 3) {
+#pragma unroll
+        for (int g = 0; g < B::G; ++g) nx[g] = rd[16 * (t + 1) * B::XS + 4 * g];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      int q = 0;
+#pragma unroll
+      for (int g = 0; g < B::G; ++g)
+#pragma unroll
+        for (int h = g; h < B::G; ++h, ++q) acc[q] = mfma_4b(x[g], x[h], acc[q]);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
 
 // Deepest ring (<= PQ_NBUF buffers) whose chunks (nv doubles per point), the
 // headers, the producers' record copies (rec_lds) and, with the matrix-core
 // Gram, the transposition tiles fit the LDS.
 constexpr int pq_ring_depth(int nv, bool mx, bool rec_lds) {
   int nb = PQ_NBUF;
-  while (nb > 2 && PC_EPB * (nb * (nv * 64 * 8 + 16) + 8 + (mx ? 64 * PQ_XS * 8 : 0) + (rec_lds ? REC_SITE * 8 : 0)) >
+  while (nb > 2 && PC_EPB * (nb * (nv * 64 * 8 + 16) + 8 + (mx ? PQ_TILE * 8 : 0) + (rec_lds ? REC_SITE * 8 : 0)) >
                        PQ_LDS_BYTES)
     --nb;
   return nb;
 }
-#ifndef GWF_PQ_NACC
-#define GWF_PQ_NACC 2  // measured: 4 accumulators no faster
-#endif
-constexpr int PQ_NACC = GWF_PQ_NACC;
-
-template <int P, int NA = PQ_NACC>
-__device__ __forceinline__ void mfma_rows(const double* re, const double* im, double* X, int lane, v4d* acc) {
-  const int rd = (lane >> 4) * PQ_XS + (lane & 15);
-#pragma unroll
-  for (int part = 0; part < 2; ++part) {
-    const double* v = part ? im : re;
-#pragma unroll
-    for (int i = 0; i < P; ++i) X[lane * PQ_XS + i] = v[i];
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const double x = X[4 * t * PQ_XS + rd];
-      acc[t % NA] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, x, acc[t % NA], 0, 0, 0);
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-}
-
 // Consumer with every Gram update on the matrix cores (mfma_rows); dead lanes
 // (points past res) take part with zero rows.  MODE PQ_SUM: the network-sum
-// arms into acc[0..PQ_NACC); PQ_MASKED: the arms whose bit is set in mask, a
-// site with all arms set through its sum arms; PQ_ARMS: physical arm a alone
-// into acc[a] (a < PQ_ARMS_MAX), for the per-arm Fisher matrices.
+// arms; PQ_MASKED: the arms whose bit is set in mask, a site with all arms set
+// through its sum arms; PQ_ARMS: physical arm a alone into accumulators
+// [a * ACCS, (a + 1) * ACCS) (a < PQ_ARMS_MAX), for the per-arm Fisher
+// matrices.
 constexpr int PQ_SUM = 0, PQ_MASKED = 1, PQ_ARMS = 2;
 constexpr int PQ_ARMS_MAX = 8;
 template <int MODEL, int NT, int P, int MODE>
 __device__ __forceinline__ void pc_consume_mx(const NetK& net, const double* rec, int base, int res, int lane,
-                                              const double* buf, double* X, v4d* acc, uint32_t mask) {
+                                              const double* buf, double* X, double* acc, uint32_t mask) {
   typedef PcLayout<NT> L;
   __asm__ volatile("" ::: "memory");
   const bool live = base + lane < res;
@@ -293,8 +364,14 @@ __device__ __forceinline__ void pc_consume_mx(const NetK& net, const double* rec
       double Ap, Ac;
       arm_derivs<MODEL, NT, P>(wp, ev, sc, g, arm, S.motion, f, re, im, &Ap, &Ac, sw * arm.swgt);
     } else {
+      // (re before im, as arm_derivs stores them: the other way round the
+      // compiler merges the branches' last stores into one through a pointer,
+      // which keeps that element of both arrays in scratch memory)
 #pragma unroll
-      for (int i = 0; i < P; ++i) re[i] = im[i] = 0.0;
+      for (int i = 0; i < P; ++i) {
+        re[i] = 0.0;
+        im[i] = 0.0;
+      }
     }
   };
   if constexpr (MODE == PQ_ARMS) {
@@ -304,7 +381,7 @@ __device__ __forceinline__ void pc_consume_mx(const NetK& net, const double* rec
       if (a < net.n_arms) {
         double re[P], im[P];
         arm_rows(net.arm[a], net.arm[a].site, re, im);
-        mfma_rows<P, 1>(re, im, X, lane, acc + a);
+        mfma_rows<P>(re, im, X, lane, acc + a * GramBlocks<P>::ACCS);
       }
     }
   } else if constexpr (MODE == PQ_MASKED) {
@@ -340,14 +417,13 @@ __device__ __forceinline__ void pc_consume_mx(const NetK& net, const double* rec
 // Re(c_p conj(c_q)) W.  On the matrix cores: the pure x other entries
 // sum_points (c_pr Tr_j - c_pi Ti_j) -- per chunk each lane writes its
 // point's [c_r | Tr] and then [-c_i | Ti] into the wave's LDS tile (pure
-// factors in columns 0..NPU-1, T in 8..14) and 16 v_mfma_f64_16x16x4f64 per
-// part contract over the 64 points (A[p][k] = tile[4t + k][p],
-// B[k][j] = tile[4t + k][8 + j]; D[p][j] in lane j + 16 (p % 4), item p / 4).
-// 32 MFMAs per chunk instead of 32 per arm.  G holds the 28 entries of the
-// 7 rows (packed, pk<7>) and then the pure x pure ones (pk<NPU>).
+// factors in columns 0..NPU-1, T in 8..14) and the 2 x 2 block pairs of
+// factors and sums contract over the 64 points (acc[2 g + h]: factors 4g..,
+// sums 4h..).  G holds the 28 entries of the 7 rows (packed, pk<7>) and then
+// the pure x pure ones (pk<NPU>).
 template <int MODEL, int NT, int P>
 __device__ __forceinline__ void pc_consume_pure_mx(const NetK& net, const double* rec, int base, int res, int lane,
-                                                    const double* buf, double* X, double* G, v4d& acc) {
+                                                    const double* buf, double* X, double* G, double* acc) {
   constexpr int NPU = P - 7;
   static_assert(NPU >= 2 && NPU <= 8, "pure rows: dL, Phicoal and up to six waveform-only rows");
   typedef PcLayout<NT> L;
@@ -423,28 +499,36 @@ __device__ __forceinline__ void pc_consume_pure_mx(const NetK& net, const double
         x = fma(fma(cr[p], cr[q], ci[p] * ci[q]), W, x);
       }
   }
-  const int rd = (lane >> 4) * PQ_XS;
+  constexpr int XS = pq_pitch(4);
+  const double* rd = tile_at<XS>(X, lane);
+  double2* row = (double2*)(X + lane * XS);
 #pragma unroll
   for (int part = 0; part < 2; ++part) {
+    auto c = [&](int p) { return p < NPU ? (part ? -ci[p] : cr[p]) : 0.0; };
+    auto T = [&](int j) { return j < 7 ? (part ? Ti[j] : Tr[j]) : 0.0; };
 #pragma unroll
-    for (int p = 0; p < NPU; ++p) X[lane * PQ_XS + p] = part ? -ci[p] : cr[p];
+    for (int p = 0; p < 8; p += 2) row[p / 2] = make_double2(c(p), c(p + 1));
 #pragma unroll
-    for (int j = 0; j < 7; ++j) X[lane * PQ_XS + 8 + j] = part ? Ti[j] : Tr[j];
+    for (int j = 0; j < 8; j += 2) row[4 + j / 2] = make_double2(T(j), T(j + 1));
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const double a = X[4 * t * PQ_XS + rd + (lane & 15)];
-      const double b = X[4 * t * PQ_XS + rd + 8 + (lane & 7)];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+    for (int t = 0; t < 4; ++t) {
+      double x[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) x[g] = rd[16 * t * XS + 4 * g];
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) acc[2 * g + h] = mfma_4b(x[g], x[2 + h], acc[2 * g + h]);
     }
     __builtin_amdgcn_wave_barrier();
   }
 }
 
 // Stores the Fisher of pc_consume_pure_mx: the VALU entries wave-reduced,
-// the pure x other entries from the matrix-core accumulator.
+// the pure x other entries from the matrix-core accumulators.
 template <int P>
-__device__ __forceinline__ void store_pure_mx(const double* G, const v4d& acc, double* __restrict__ F, int64_t n_ev,
+__device__ __forceinline__ void store_pure_mx(const double* G, const double* acc, double* __restrict__ F, int64_t n_ev,
                                               int64_t e, int lane) {
   constexpr int NPU = P - 7;
   constexpr int NP[7] = {0, 1, 3, 4, 5, 6, 7};
@@ -468,12 +552,14 @@ __device__ __forceinline__ void store_pure_mx(const double* G, const v4d& acc, d
       const double s = wave_sum(G[28 + pk<NPU>(p, q)]);
       if (lane == (k & 63)) put(PU(p), PU(q), s);
     }
-  const int j = lane & 15;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int p = (lane >> 4) + 4 * r;
-    if (p < NPU && j < 7) put(PU(p), NP[j], acc[r]);
-  }
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const double v = block_sum(acc[2 * g + h]);
+      const int p = 4 * g + (lane >> 4), j = 4 * h + (lane & 3);
+      if ((lane & 12) == 0 && p < NPU && j < 7) put(PU(p), NP[j], v);
+    }
 }
 
 // Consumer for 12-14 parameters with the Mc, eta and tcoal rows factored as
@@ -484,8 +570,11 @@ __device__ __forceinline__ void store_pure_mx(const double* G, const v4d& acc, d
 // point's 3 x 3 of the W sums, and s_j Tv_k of the three rows with s_j != 0.
 // On the matrix cores: the rest of the sky x factored entries,
 // sum_points (Re c_j Tr_k - Im c_j Ti_k), per chunk through the wave's LDS
-// tile ([Re c | Tr], then [-Im c | Ti]: c in columns 0..NF-1, T in 10..13)
-// with 32 v_mfma_f64_16x16x4f64, as pc_consume_pure_mx.
+// tile ([Re c | Tr], then [-Im c | Ti]: c in the first groups, T in the last)
+// with one 4 x 4 block product per group of 4 factors and 16 points.
+// Against the same sums in 16 x 16 tiles (32 MFMAs of 64 cycles a chunk, most
+// of them on padding): tidal TaylorF2, 2 x 10^4 ragged events of 500..10^4
+// points 8.94 -> 8.06 ms, 5000 NRTidalv2 events x 1000 points 623 -> 579 us.
 template <int P>
 __device__ __forceinline__ constexpr int semi_row(int j) {  // factored row j: 0, 1, 7, 2, 8, 9, ..., P-1
   return j < 3 ? (j == 2 ? 7 : j) : (j == 3 ? 2 : 4 + j);
@@ -495,7 +584,7 @@ __device__ __forceinline__ constexpr bool semi_hi(int j) { return j != 3; }     
 __device__ __forceinline__ constexpr bool semi_hs(int j) { return j < 3; }             // s_j not identically 0
 template <int MODEL, int NT, int P, bool MASKED = false>
 __device__ __forceinline__ void pc_consume_semi_vx(const NetK& net, const double* rec, int base, int res, int lane,
-                                                    const double* buf, double* X, double* G, v4d& acc,
+                                                    const double* buf, double* X, double* G, double* acc,
                                                     uint32_t mask = 0u) {
   constexpr int NF = P - 4;
   constexpr int NFF = NF * (NF + 1) / 2;  // G: [factored x factored | s x sky (12) | sky x sky (10)]
@@ -630,27 +719,35 @@ __device__ __forceinline__ void pc_consume_semi_vx(const NetK& net, const double
     }
   }
   // sum_points (Re c_j Tr_k - Im c_j Ti_k) on the matrix cores
-  const int rd = (lane >> 4) * PQ_XS;
+  constexpr int GC = (NF + 3) / 4, XS = pq_pitch(GC + 1);
+  const double* rd = tile_at<XS>(X, lane);
+  double2* row = (double2*)(X + lane * XS);
 #pragma unroll
   for (int part = 0; part < 2; ++part) {
+    auto c = [&](int j) { return j < NF ? (part ? -ci[j < NF ? j : 0] : cr[j < NF ? j : 0]) : 0.0; };
+    const double* T = part ? Ti : Tr;
 #pragma unroll
-    for (int j = 0; j < NF; ++j) X[lane * PQ_XS + j] = part ? -ci[j] : cr[j];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) X[lane * PQ_XS + 10 + a] = part ? Ti[a] : Tr[a];
+    for (int j = 0; j < 4 * GC; j += 2) row[j / 2] = make_double2(c(j), c(j + 1));
+    row[2 * GC] = make_double2(T[0], T[1]);
+    row[2 * GC + 1] = make_double2(T[2], T[3]);
     __builtin_amdgcn_wave_barrier();
+    double x[4][GC + 1];  // every read before the first product
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const double a = X[4 * t * PQ_XS + rd + (lane & 15)];
-      const double b = X[4 * t * PQ_XS + rd + 10 + (lane & 3)];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-    }
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int g = 0; g <= GC; ++g) x[t][g] = rd[16 * t * XS + 4 * g];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int g = 0; g < GC; ++g) acc[g] = mfma_4b(x[t][g], x[t][GC], acc[g]);
     __builtin_amdgcn_wave_barrier();
   }
 }
 
 // Stores the Fisher of pc_consume_semi_vx.
 template <int P>
-__device__ __forceinline__ void store_semi_vx(const double* G, const v4d& acc, double* __restrict__ F, int64_t n_ev,
+__device__ __forceinline__ void store_semi_vx(const double* G, const double* acc, double* __restrict__ F, int64_t n_ev,
                                               int64_t e, int lane) {
   constexpr int NF = P - 4, NFF = NF * (NF + 1) / 2;
   constexpr int SK[4] = {3, 4, 5, 6};
@@ -673,17 +770,17 @@ __device__ __forceinline__ void store_semi_vx(const double* G, const v4d& acc, d
       const double s = wave_sum(G[NFF + 12 + pk<4>(a, b)]);
       if (lane == ((NFF + pk<4>(a, b)) & 63)) put(SK[a], SK[b], s);
     }
-  // sky x factored: the matrix-core part (element (j, k) in lane k + 16 (j % 4),
-  // item j / 4) plus, for the rows with s_j != 0, the wave sum of s_j Tv_k
+  // sky x factored: the matrix-core part (element (j, k) in lane k + 16 (j % 4)
+  // of group j / 4) plus, for the rows with s_j != 0, the wave sum of s_j Tv_k
   double st[12];
 #pragma unroll
   for (int i = 0; i < 12; ++i) st[i] = wave_sum(G[NFF + i]);
-  const int k = lane & 15;
+  const int k = lane & 3;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
+  for (int r = 0; r < (NF + 3) / 4; ++r) {
     const int j = (lane >> 4) + 4 * r;
-    if (j < NF && k < 4) {
-      double v = acc[r];
+    double v = block_sum(acc[r]);
+    if (j < NF && (lane & 12) == 0) {
 #pragma unroll
       for (int jj = 0; jj < 3; ++jj)
 #pragma unroll
@@ -694,23 +791,34 @@ __device__ __forceinline__ void store_semi_vx(const double* G, const v4d& acc, d
   }
 }
 
-// Stores the event's Fisher from the NACC matrix-core accumulators (element
-// (i, j) in lane j + 16 (i % 4), item i / 4): the upper-triangle element
-// (i <= j) goes to both F[i][j] and F[j][i].
-template <int P, int NA = PQ_NACC>
-__device__ __forceinline__ void store_mx(const v4d* acc, double* __restrict__ F, int64_t n_ev, int64_t e, int lane) {
-  const int j = lane & 15;
+// Stores the event's Fisher from the block-pair accumulators of mfma_rows:
+// the upper-triangle element (i <= j) goes to both F[i][j] and F[j][i].
+template <int P>
+__device__ __forceinline__ void store_mx(const double* acc, double* __restrict__ F, int64_t n_ev, int64_t e, int lane) {
+  if constexpr (GramBlocks<P>::G == 4) {
+    const int j = lane & 15;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int i = (lane >> 4) + 4 * r;
-    double v = 0.0;
-#pragma unroll
-    for (int q = 0; q < NA; ++q) v += acc[q][r];
-    if (i < P && j < P && i <= j) {
-      F[(int64_t)(i * P + j) * n_ev + e] = v;
-      if (i != j) F[(int64_t)(j * P + i) * n_ev + e] = v;
+    for (int r = 0; r < 4; ++r) {
+      const int i = (lane >> 4) + 4 * r;
+      if (i < P && j < P && i <= j) {
+        F[(int64_t)(i * P + j) * n_ev + e] = acc[r];
+        if (i != j) F[(int64_t)(j * P + i) * n_ev + e] = acc[r];
+      }
     }
+    return;
   }
+  int q = 0;
+#pragma unroll
+  for (int g = 0; g < GramBlocks<P>::G; ++g)
+#pragma unroll
+    for (int h = g; h < GramBlocks<P>::G; ++h, ++q) {
+      const double v = block_sum(acc[q]);
+      const int i = 4 * g + (lane >> 4), j = 4 * h + (lane & 3);
+      if ((lane & 12) == 0 && i < P && j < P && i <= j) {
+        F[(int64_t)(i * P + j) * n_ev + e] = v;
+        if (i != j) F[(int64_t)(j * P + i) * n_ev + e] = v;
+      }
+    }
 }
 
 // Models with at least GWF_PQ_MFMA_MIN_P parameters take the matrix-core Gram
@@ -786,7 +894,7 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
   __shared__ double buf[PC_EPB][NB][L::NV * 64];
   __shared__ int head[PC_EPB][NB][4];  // event, chunk, grid length of the item in each buffer
   __shared__ int cnt[PC_EPB][2];            // items produced, items consumed
-  __shared__ double xt[PC_EPB][MX ? 64 * PQ_XS : 1];  // consumers' transposition tiles
+  __shared__ __align__(16) double xt[PC_EPB][MX ? PQ_TILE : 2];  // consumers' transposition tiles
   // each producer's copy of its event's waveform slots and event constants
   // (3.9 KB): read per chunk from LDS instead of through the scalar cache,
   // which the four pairs' records (5.6 KB each, both waves reading) thrash
@@ -853,20 +961,19 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
     }
   } else if constexpr (MX && MODE == PQ_SUM && PURE_MX) {  // rows factored out, see pc_consume_semi_vx
     double* X = xt[slot];
-    for (int q = lane; q < 64 * PQ_XS; q += 64) X[q] = 0.0;
 #ifndef GWF_NO_SEMI_ROWS
     // the Mc, eta, tcoal rows factored as well, up to 13 parameters (at 14
     // the consumer spills 88 VGPRs: 2.44 -> 3.07 ms per 10^4 events)
     if (SEMI_VX && !net.mixed_motion) {
       constexpr int NF = P - 4, NG = NF * (NF + 1) / 2 + 12 + 10;
-      double G[NG];
-      v4d acc;
+      double G[NG], acc[(NF + 3) / 4];
       pq_consumer<NB>(&cnt[slot][0], &cnt[slot][1], head[slot], buf[slot], counter, net.spin_limit, lane,
                       [&](int e, int t, int res, const double* chunk) {
                         if (t == 0) {
 #pragma unroll
                           for (int q = 0; q < NG; ++q) G[q] = 0.0;
-                          acc = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                          for (int q = 0; q < (NF + 3) / 4; ++q) acc[q] = 0.0;
                         }
                         pc_consume_semi_vx<MODEL, NT, P>(net, rec + (int64_t)e * REC_DOUBLES, t * 64, res, lane,
                                                          chunk, X, G, acc);
@@ -876,14 +983,14 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
     }
 #endif
     constexpr int NPU = P - 7, NG = 28 + NPU * (NPU + 1) / 2;
-    double G[NG];
-    v4d acc;
+    double G[NG], acc[4];
     pq_consumer<NB>(&cnt[slot][0], &cnt[slot][1], head[slot], buf[slot], counter, net.spin_limit, lane,
                     [&](int e, int t, int res, const double* chunk) {
                       if (t == 0) {
 #pragma unroll
                         for (int q = 0; q < NG; ++q) G[q] = 0.0;
-                        acc = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) acc[q] = 0.0;
                       }
                       pc_consume_pure_mx<MODEL, NT, P>(net, rec + (int64_t)e * REC_DOUBLES, t * 64, res, lane, chunk,
                                                        X, G, acc);
@@ -891,19 +998,19 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
                     [&](int e) { store_pure_mx<P>(G, acc, F, n_ev, e, lane); });
   } else if constexpr (MX) {  // Gram on the matrix cores
     double* X = xt[slot];
-    for (int q = lane; q < 64 * PQ_XS; q += 64) X[q] = 0.0;  // padding columns stay zero
+    for (int q = lane; q < PQ_TILE; q += 64) X[q] = 0.0;  // padding columns stay zero
     if constexpr (SEMI_VX_M) {  // masked network sum, rows factored as in the unmasked one
       if (!net.mixed_motion) {
         constexpr int NF = P - 4, NG = NF * (NF + 1) / 2 + 12 + 10;
-        double G[NG];
-        v4d acc1;
+        double G[NG], acc1[(NF + 3) / 4];
         uint32_t mask = 0u;
         pq_consumer<NB>(&cnt[slot][0], &cnt[slot][1], head[slot], buf[slot], counter, net.spin_limit, lane,
                         [&](int e, int t, int res, const double* chunk) {
                           if (t == 0) {
 #pragma unroll
                             for (int q = 0; q < NG; ++q) G[q] = 0.0;
-                            acc1 = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                            for (int q = 0; q < (NF + 3) / 4; ++q) acc1[q] = 0.0;
                             mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)arm_mask[e]);
                           }
                           pc_consume_semi_vx<MODEL, NT, P, true>(net, rec + (int64_t)e * REC_DOUBLES, t * 64, res,
@@ -913,14 +1020,14 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
         return;
       }
     }
-    constexpr int NA = ARMS ? PQ_ARMS_MAX : PQ_NACC;        // ARMS: one accumulator per physical arm
-    v4d acc[NA];
+    constexpr int NB2 = GramBlocks<P>::ACCS, NA = ARMS ? PQ_ARMS_MAX * NB2 : NB2;  // ARMS: a set per physical arm
+    double acc[NA];
     uint32_t mask = 0u;
     pq_consumer<NB>(&cnt[slot][0], &cnt[slot][1], head[slot], buf[slot], counter, net.spin_limit, lane,
                     [&](int e, int t, int res, const double* chunk) {
                       if (t == 0) {
 #pragma unroll
-                        for (int q = 0; q < NA; ++q) acc[q] = v4d{0.0, 0.0, 0.0, 0.0};
+                        for (int q = 0; q < NA; ++q) acc[q] = 0.0;
                         if (MASKED) mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)arm_mask[e]);
                       }
                       pc_consume_mx<MODEL, NT, P, MODE>(net, rec + (int64_t)e * REC_DOUBLES, t * 64, res, lane, chunk,
@@ -930,7 +1037,8 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
                       if constexpr (ARMS) {  // F: (n_arms, P, P, n_ev)
 #pragma unroll
                         for (int a = 0; a < PQ_ARMS_MAX; ++a)
-                          if (a < net.n_arms) store_mx<P, 1>(acc + a, F + (int64_t)a * P * P * n_ev, n_ev, e, lane);
+                          if (a < net.n_arms)
+                            store_mx<P>(acc + a * NB2, F + (int64_t)a * P * P * n_ev, n_ev, e, lane);
                       } else {
                         store_mx<P>(acc, F, n_ev, e, lane);
                       }
