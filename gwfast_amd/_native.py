@@ -106,6 +106,10 @@ SIGNATURES = {
     'gwf_head_forward': (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
     'gwf_head_backward': (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p,
                                          c_void_p]),
+    'gwf_mlp_forward': (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_int64] + [c_void_p] * 8),
+    'gwf_mlp_backward_workspace_bytes': (ctypes.c_size_t, [c_int64]),
+    'gwf_mlp_backward': (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64] + [c_void_p] * 8
+                         + [ctypes.c_size_t, c_void_p]),
     'gwf_mse_grad': (ctypes.c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
     'gwf_adam': (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_float, c_float, c_float, c_float,
                                 c_int32, c_void_p, c_void_p]),

@@ -16,6 +16,9 @@
 //   gwf_mse_grad       loss and dL/dy of the mean squared error
 //   gwf_adam           Adam on fp32 master weights + bf16 copies
 //   gwf_snr_features   event parameters -> standardised features
+//   gwf_mlp_forward    the whole network on standardised features, activations
+//                      kept for the backward pass
+//   gwf_mlp_backward   every gradient of sum(g y), from those activations
 // Inference: gwf_snr_screen runs features + the whole MLP + the threshold
 // decision in one launch (128 events per workgroup, activations in LDS,
 // weights from L2, v_mfma_f32_16x16x32_bf16 for the 256-wide layers).
@@ -293,6 +296,365 @@ __global__ void k_features(const double* __restrict__ par, int64_t ld, int64_t n
   if (X)
 #pragma unroll
     for (int k = NFEAT; k < KFEAT; ++k) X[e * KFEAT + k] = 0;
+}
+
+// ------------------------------------------------- fused training passes
+// Forward and backward of the whole network on a batch of B rows: at the
+// training sizes (256 to 8192 rows) the work is 2-7 GFLOP and a few MB, so
+// what bounds it is the number of launches and the serial chains in each.
+// As 31 launches of the kernels above 440 us per forward + backward of 4096
+// rows (the column sums alone ten launches of 18-90 us each); as
+// k_mlp_fwd, k_mlp_bwd, k_mlp_dw and k_mlp_reduce 71 us (25, 19, 23 and 4).
+//
+// k_mlp_fwd / k_mlp_bwd: 16 rows per workgroup (4096 rows = 256 workgroups,
+// one per CU), wave w owns the 64 columns 64 w.. in four MFMA tiles; tile j
+// holds the columns 64 w + 4 c + j (c = lane % 16), so a lane's four tiles
+// are four neighbouring columns and every load and store of activations is
+// 8 or 16 bytes wide.  The weights come from L2 straight into registers, a
+// whole layer's 64 fragments per lane requested before the layer before it
+// is finished.  The products run through v_mfma_f32_16x16x16_bf16 in k order
+// as gwf_gemm_bf16, and the elementwise formulas are those of k_bias_silu and
+// k_silu_bwd, so y, Z, H and the bf16 dZ are the same numbers.
+struct MlpParams {  // flat parameter layout: W1 (256, 16), W2, W3 (256, 256), b1, b2, b3, w4 (256), b4 (1)
+  static constexpr int W1 = 0, W2 = W1 + HID * KFEAT, W3 = W2 + HID * HID, B1 = W3 + HID * HID, B2 = B1 + HID,
+                       B3 = B2 + HID, W4 = B3 + HID, B4 = W4 + HID, N = B4 + 1;
+};
+constexpr int TR_ROWS = 16;         // rows per workgroup of k_mlp_fwd / k_mlp_bwd
+constexpr int TR_LD = HID + 8;      // LDS row stride (bf16 elements)
+constexpr int BSUM = 4 * HID + 4;   // per-workgroup column sums: b1, b2, b3, w4, then b4 and three pads
+
+struct MlpActs {  // activations of a batch: Z fp32, H and dZ bf16, each (B, 256)
+  float* Z[3];
+  uint16_t* H[3];
+  uint16_t* dZ[3];
+};
+
+// acc[j] += A B_j over K = 256, A(row r16, k) from LDS, B_j from b[step][j]
+__device__ __forceinline__ void tr_product(const uint16_t* A, int lane, const uint2 (&b)[HID / 16][4], f32x4 (&acc)[4]) {
+  const uint16_t* a0 = A + (lane & 15) * TR_LD + 4 * (lane >> 4);
+#pragma unroll
+  for (int s = 0; s < HID / 16; ++s) {
+    const bf16x4 a = __builtin_bit_cast(bf16x4, *(const uint2*)(a0 + 16 * s));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, __builtin_bit_cast(bf16x4, b[s][j]), acc[j], 0, 0, 0);
+  }
+}
+
+__device__ __forceinline__ uint2 pack4(const float* v) {
+  return make_uint2((uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16), (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
+}
+
+__global__ __launch_bounds__(256, 1) void k_mlp_fwd(const uint16_t* __restrict__ X, const uint16_t* __restrict__ wb,
+                                                    const float* __restrict__ wf, int64_t M, MlpActs act,
+                                                    float* __restrict__ y) {
+  __shared__ __align__(16) uint16_t Hs[2][TR_ROWS * TR_LD];  // two tiles: a layer reads one and writes the other
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, q = lane >> 4;
+  const int col = 64 * wave + 4 * c;  // tile j: column col + j
+  const int64_t m0 = (int64_t)blockIdx.x * TR_ROWS;
+  uint2 b[HID / 16][4];
+  auto load_w = [&](int off) {
+#pragma unroll
+    for (int s = 0; s < HID / 16; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[s][j] = *(const uint2*)(wb + off + (col + j) * HID + 16 * s + 4 * q);
+  };
+  f32x4 acc[4];
+  {  // first layer, K = 16: one step
+    bf16x4 x = {0, 0, 0, 0};
+    if (m0 + c < M) {
+      const uint16_t* xr = X + (m0 + c) * KFEAT + 4 * q;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = (short)xr[i];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const bf16x4 w1 = __builtin_bit_cast(bf16x4, *(const uint2*)(wb + MlpParams::W1 + (col + j) * KFEAT + 4 * q));
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, w1, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    }
+  }
+  // bias, SiLU; Z and H to memory, H to LDS
+  auto epilogue = [&](int l, int boff) {
+    const float4 bias = *(const float4*)(wf + boff + col);
+    const float bj[4] = {bias.x, bias.y, bias.z, bias.w};
+    uint16_t* hs = Hs[l & 1];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 4 * q + r;
+      float z[4], h[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        z[j] = acc[j][r] + bj[j];
+        h[j] = silu(z[j]);
+      }
+      const uint2 hb = pack4(h);
+      *(uint2*)(hs + row * TR_LD + col) = hb;
+      if (m0 + row < M) {
+        *(float4*)(act.Z[l] + (m0 + row) * HID + col) = make_float4(z[0], z[1], z[2], z[3]);
+        *(uint2*)(act.H[l] + (m0 + row) * HID + col) = hb;
+      }
+    }
+  };
+  load_w(MlpParams::W2);
+  __builtin_amdgcn_sched_barrier(0);
+  epilogue(0, MlpParams::B1);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  tr_product(Hs[0], lane, b, acc);
+  load_w(MlpParams::W3);
+  __builtin_amdgcn_sched_barrier(0);
+  epilogue(1, MlpParams::B2);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  tr_product(Hs[1], lane, b, acc);
+  epilogue(2, MlpParams::B3);
+  __syncthreads();
+  // y = H3 w4 + b4, one wave per row, in k_head_fwd's order
+#pragma unroll
+  for (int i = 0; i < TR_ROWS / 4; ++i) {
+    const int row = wave + 4 * i;
+    float s = 0.f;
+#pragma unroll
+    for (int p = 0; p < HID / 64; ++p) s += bf2f(Hs[0][row * TR_LD + p * 64 + lane]) * wf[MlpParams::W4 + p * 64 + lane];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0 && m0 + row < M) y[m0 + row] = s + wf[MlpParams::B4];
+  }
+}
+
+// operand of tile j, rows k..k+3 of a row-major matrix read four columns wide
+__device__ __forceinline__ bf16x4 column_of(const uint2* r, int j) {
+  bf16x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = (short)((j & 2 ? r[i].y : r[i].x) >> (j & 1 ? 16 : 0));
+  return o;
+}
+
+__global__ __launch_bounds__(256, 1) void k_mlp_bwd(const uint16_t* __restrict__ wb, const float* __restrict__ wf,
+                                                    const float* __restrict__ g, int64_t M, MlpActs act,
+                                                    float* __restrict__ bsum) {
+  __shared__ __align__(16) uint16_t Ds[2][TR_ROWS * TR_LD];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, q = lane >> 4;
+  const int col = 64 * wave + 4 * c;
+  const int64_t m0 = (int64_t)blockIdx.x * TR_ROWS;
+  float* bs = bsum + (int64_t)blockIdx.x * BSUM;
+  uint2 b[HID / 16][4];  // b[s][i]: row 16 s + 4 q + i of W, columns col..col+3
+  auto load_w = [&](int off) {
+#pragma unroll
+    for (int s = 0; s < HID / 16; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[s][i] = *(const uint2*)(wb + off + (16 * s + 4 * q + i) * HID + col);
+  };
+  // sums of v over the workgroup's rows: the lane's four rows are in v already
+  auto column_sums = [&](float* v, int off) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[j] += __shfl_xor(v[j], 16);
+      v[j] += __shfl_xor(v[j], 32);
+    }
+    if (q == 0) *(float4*)(bs + off + col) = make_float4(v[0], v[1], v[2], v[3]);
+  };
+  load_w(MlpParams::W3);
+  __builtin_amdgcn_sched_barrier(0);
+  float dh[4][4];  // dH of (row 4 q + r, column col + j)
+  {                // output layer: dH3 = g w4^T, dw4 = H3^T g, db4 = sum g
+    const float4 w4 = *(const float4*)(wf + MlpParams::W4 + col);
+    const float wj[4] = {w4.x, w4.y, w4.z, w4.w};
+    float dw[4] = {0.f, 0.f, 0.f, 0.f}, dg = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t m = m0 + 4 * q + r;
+      const float gm = m < M ? g[m] : 0.f;
+      uint2 h = make_uint2(0u, 0u);
+      if (m < M) h = *(const uint2*)(act.H[2] + m * HID + col);
+      const float hj[4] = {bf2f((uint16_t)h.x), bf2f((uint16_t)(h.x >> 16)), bf2f((uint16_t)h.y), bf2f((uint16_t)(h.y >> 16))};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        dh[r][j] = gm * wj[j];
+        dw[j] += gm * hj[j];
+      }
+      dg += gm;
+    }
+    column_sums(dw, 3 * HID);
+    dg += __shfl_xor(dg, 16);
+    dg += __shfl_xor(dg, 32);
+    if (threadIdx.x < 4) bs[4 * HID + threadIdx.x] = threadIdx.x == 0 ? dg : 0.f;
+  }
+#pragma unroll
+  for (int l = 2; l >= 0; --l) {
+    uint16_t* ds = Ds[l & 1];
+    float db[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 4 * q + r;
+      const bool live = m0 + row < M;
+      float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (live) z4 = *(const float4*)(act.Z[l] + (m0 + row) * HID + col);
+      const float z[4] = {z4.x, z4.y, z4.z, z4.w};
+      float d[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float s = 1.f / (1.f + __expf(-z[j]));
+        d[j] = live ? dh[r][j] * (s * (1.f + z[j] * (1.f - s))) : 0.f;
+        db[j] += d[j];
+      }
+      const uint2 db4 = pack4(d);
+      if (l > 0) *(uint2*)(ds + row * TR_LD + col) = db4;
+      if (live) *(uint2*)(act.dZ[l] + (m0 + row) * HID + col) = db4;
+    }
+    column_sums(db, l * HID);
+    if (l > 0) {  // dH of the layer below = dZ W
+      __syncthreads();
+      f32x4 acc[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const uint16_t* a0 = ds + c * TR_LD + 4 * q;
+#pragma unroll
+      for (int s = 0; s < HID / 16; ++s) {
+        const bf16x4 a = __builtin_bit_cast(bf16x4, *(const uint2*)(a0 + 16 * s));
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, column_of(b[s], j), acc[j], 0, 0, 0);
+      }
+      if (l == 2) {
+        load_w(MlpParams::W2);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dh[r][j] = acc[j][r];
+    }
+  }
+}
+
+// Weight gradients dW = dZ^T H of the three layers in one launch: a workgroup
+// takes a 64 x 64 block of one of them (64 x 16 of W1's) and one of `splits`
+// ranges of the batch, its four waves every fourth 16 rows of the range; both
+// operands are read four columns wide and transposed in registers.  The
+// ranges' partial sums go to part (splits, MlpParams::B1), summed in order by
+// k_mlp_reduce: no atomics, so equal inputs give equal gradients.
+constexpr int DW_BLOCKS = 36;  // 16 of W3, 16 of W2, 4 of W1
+constexpr int DW_SPLIT_ROWS = 512, DW_MAX_SPLITS = 32;  // 4096 rows: 8 ranges, 288 workgroups
+__global__ __launch_bounds__(256) void k_mlp_dw(const uint16_t* __restrict__ X, int64_t M, int64_t rows, MlpActs act,
+                                                float* __restrict__ part) {
+  __shared__ __align__(16) float red[4][64 * 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, q = lane >> 4;
+  const int t = blockIdx.x;
+  const int l = t < 16 ? 2 : (t < 32 ? 1 : 0);
+  const int i0 = 64 * (l ? (t & 15) >> 2 : t & 3), j0 = l ? 64 * (t & 3) : 0;
+  const uint16_t* D = act.dZ[l] + i0 + 4 * c;
+  const uint16_t* H = l ? act.H[l - 1] + j0 + 4 * c : X + c;
+  const int64_t mb = (int64_t)blockIdx.y * rows, me = min(M, mb + rows);
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint2 d[4], h[4];
+  auto fetch = [&](int64_t m0) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t m = m0 + 4 * q + k;
+      d[k] = h[k] = make_uint2(0u, 0u);
+      if (m < me) {
+        d[k] = *(const uint2*)(D + m * HID);
+        if (l)
+          h[k] = *(const uint2*)(H + m * HID);
+        else
+          h[k].x = H[m * KFEAT];
+      }
+    }
+  };
+  int64_t m0 = mb + 16 * wave;
+  if (m0 < me) fetch(m0);
+  for (; m0 < me; m0 += 64) {
+    bf16x4 a[4], b[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a[j] = column_of(d, j);
+      b[j] = column_of(h, j);
+    }
+    if (m0 + 64 < me) fetch(m0 + 64);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (l || j == 0) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
+  }
+  const int w = l ? 64 : 16;  // columns of the block
+  // C of tiles (i, j): element (row 16-index 4 q + r, column c) is (4 (4 q + r) + i, 4 c + j), W1: (.., c)
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 4 * (4 * q + r) + i;
+      if (l)
+        *(float4*)(red[wave] + row * 64 + 4 * c) = make_float4(acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]);
+      else
+        red[wave][row * 16 + c] = acc[i][0][r];
+    }
+  __syncthreads();
+  const int ldw = l ? HID : KFEAT;
+  float* out = part + (int64_t)blockIdx.y * MlpParams::B1 + (l == 2 ? MlpParams::W3 : (l == 1 ? MlpParams::W2 : MlpParams::W1)) +
+               (int64_t)i0 * ldw + j0;
+  for (int k = threadIdx.x; k < 64 * w; k += 256)
+    out[(int64_t)(k / w) * ldw + k % w] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+}
+
+// grad = the partial sums of k_mlp_dw over the ranges (the first RED_W
+// workgroups) and of k_mlp_bwd over its workgroups (four columns each)
+constexpr int RED_W = MlpParams::B1 / 4 / 256;
+static_assert(MlpParams::B1 % (4 * 256) == 0, "whole workgroups of float4");
+__global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ part, int splits,
+                                                    const float* __restrict__ bsum, int64_t nblk,
+                                                    float* __restrict__ grad) {
+  if (blockIdx.x < RED_W) {
+    const int64_t k = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int p = 0; p < splits; ++p) {
+      const float4 v = *(const float4*)(part + (int64_t)p * MlpParams::B1 + k);
+      s.x += v.x;
+      s.y += v.y;
+      s.z += v.z;
+      s.w += v.w;
+    }
+    grad[k] = s.x;
+    grad[k + 1] = s.y;
+    grad[k + 2] = s.z;
+    grad[k + 3] = s.w;
+    return;
+  }
+  __shared__ float4 red[256];
+  const int k = 4 * (blockIdx.x - RED_W);  // columns k..k+3 of the BSUM sums
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int64_t b = threadIdx.x; b < nblk; b += 256) {
+    const float4 v = *(const float4*)(bsum + b * BSUM + k);
+    s.x += v.x;
+    s.y += v.y;
+    s.z += v.z;
+    s.w += v.w;
+  }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) {
+      float4 &u = red[threadIdx.x];
+      const float4 v = red[threadIdx.x + o];
+      u.x += v.x;
+      u.y += v.y;
+      u.z += v.z;
+      u.w += v.w;
+    }
+    __syncthreads();
+  }
+  const float* r = (const float*)&red[0];
+  if (threadIdx.x < 4 && k + (int)threadIdx.x <= 4 * HID) grad[MlpParams::B1 + k + threadIdx.x] = r[threadIdx.x];
 }
 
 // ------------------------------------------------------- fused screen
@@ -689,6 +1051,62 @@ int gwf_snr_screen(const double* params, int64_t ld, int64_t n_ev, const float* 
   a.class_out = class_out;
   hipLaunchKernelGGL(k_mlp_screen, dim3(blocks_for(n_ev, SCR_ROWS)), dim3(256), 0, (hipStream_t)stream, a);
   return launch_ok("gwf_snr_screen launch");
+}
+
+static int64_t mlp_blocks(int64_t B) { return (B + TR_ROWS - 1) / TR_ROWS; }
+static int mlp_splits(int64_t B) {
+  const int64_t n = (B + DW_SPLIT_ROWS - 1) / DW_SPLIT_ROWS;
+  return (int)(n > DW_MAX_SPLITS ? DW_MAX_SPLITS : n);
+}
+static bool misaligned(const void* p, int a) { return ((uintptr_t)p & (uintptr_t)(a - 1)) != 0; }
+
+int gwf_mlp_forward(const void* X, const void* theta_bf16, const float* theta, int64_t B, float* Z1, void* H1, float* Z2,
+                    void* H2, float* Z3, void* H3, float* y, void* stream) {
+  if (B < 0) return fail(-EINVAL, "invalid size");
+  if (B == 0) return 0;
+  if (!X || !theta_bf16 || !theta || !Z1 || !H1 || !Z2 || !H2 || !Z3 || !H3 || !y) return fail(-EINVAL, "NULL array");
+  if (mlp_blocks(B) > 0x7fffffff) return fail(-EINVAL, "too many rows for one call");
+  if (misaligned(theta_bf16, 16) || misaligned(theta, 16) || misaligned(Z1, 16) || misaligned(Z2, 16) ||
+      misaligned(Z3, 16) || misaligned(H1, 8) || misaligned(H2, 8) || misaligned(H3, 8))
+    return fail(-EINVAL, "parameters and activations must be 16-byte aligned");
+  MlpActs a = {{Z1, Z2, Z3}, {(uint16_t*)H1, (uint16_t*)H2, (uint16_t*)H3}, {nullptr, nullptr, nullptr}};
+  hipLaunchKernelGGL(k_mlp_fwd, dim3((unsigned)mlp_blocks(B)), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)X,
+                     (const uint16_t*)theta_bf16, theta, B, a, y);
+  return launch_ok("gwf_mlp_forward launch");
+}
+
+size_t gwf_mlp_backward_workspace_bytes(int64_t B) {
+  if (B < 1) return 0;
+  return 3 * (size_t)B * HID * sizeof(uint16_t) +
+         ((size_t)mlp_blocks(B) * BSUM + (size_t)mlp_splits(B) * MlpParams::B1) * sizeof(float);
+}
+
+int gwf_mlp_backward(const void* X, const void* theta_bf16, const float* theta, const float* g, int64_t B,
+                     const float* Z1, const void* H1, const float* Z2, const void* H2, const float* Z3, const void* H3,
+                     float* grad_out, void* workspace, size_t workspace_bytes, void* stream) {
+  if (B < 1) return fail(-EINVAL, "invalid size");
+  if (!X || !theta_bf16 || !theta || !g || !Z1 || !H1 || !Z2 || !H2 || !Z3 || !H3 || !grad_out || !workspace)
+    return fail(-EINVAL, "NULL array");
+  if (mlp_blocks(B) > 0x7fffffff) return fail(-EINVAL, "too many rows for one call");
+  if (workspace_bytes < gwf_mlp_backward_workspace_bytes(B)) return fail(-EINVAL, "workspace too small");
+  if (misaligned(theta_bf16, 16) || misaligned(theta, 16) || misaligned(workspace, 16) || misaligned(Z1, 16) ||
+      misaligned(Z2, 16) || misaligned(Z3, 16) || misaligned(H1, 8) || misaligned(H2, 8) || misaligned(H3, 8))
+    return fail(-EINVAL, "parameters, activations and workspace must be 16-byte aligned");
+  hipStream_t s = (hipStream_t)stream;
+  uint16_t* dz = (uint16_t*)workspace;
+  float* bsum = (float*)(dz + 3 * B * HID);
+  float* part = bsum + mlp_blocks(B) * BSUM;
+  MlpActs a = {{const_cast<float*>(Z1), const_cast<float*>(Z2), const_cast<float*>(Z3)},
+               {(uint16_t*)H1, (uint16_t*)H2, (uint16_t*)H3},
+               {dz, dz + B * HID, dz + 2 * B * HID}};
+  const int splits = mlp_splits(B);
+  const int64_t rows = ((B + splits - 1) / splits + 63) / 64 * 64;
+  hipLaunchKernelGGL(k_mlp_bwd, dim3((unsigned)mlp_blocks(B)), dim3(256), 0, s, (const uint16_t*)theta_bf16, theta, g, B,
+                     a, bsum);
+  hipLaunchKernelGGL(k_mlp_dw, dim3(DW_BLOCKS, (unsigned)splits), dim3(256), 0, s, (const uint16_t*)X, B, rows, a, part);
+  hipLaunchKernelGGL(k_mlp_reduce, dim3(RED_W + BSUM / 4), dim3(256), 0, s, (const float*)part, splits,
+                     (const float*)bsum, mlp_blocks(B), grad_out);
+  return launch_ok("gwf_mlp_backward launch");
 }
 
 size_t gwf_select_workspace_bytes(int64_t n) {

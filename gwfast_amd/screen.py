@@ -87,14 +87,15 @@ class _Batch:
         dev = device()
         f32, bf = T.float32, T.bfloat16
         self.B = B
-        self.C = T.empty((B, HID), dtype=f32, device=dev)
         self.Z = [T.empty((B, HID), dtype=f32, device=dev) for _ in range(3)]
         self.H = [T.empty((B, HID), dtype=bf, device=dev) for _ in range(3)]
-        self.dH = T.empty((B, HID), dtype=f32, device=dev)
-        self.dZ = T.empty((B, HID), dtype=f32, device=dev)
-        self.dZb = T.empty((B, HID), dtype=bf, device=dev)
+        self.ws = T.empty(max(16, int(N.lib().gwf_mlp_backward_workspace_bytes(B))), dtype=T.uint8, device=dev)
         self.y = T.empty(B, dtype=f32, device=dev)
         self.g = T.empty(B, dtype=f32, device=dev)
+
+    def acts(self):
+        """Z1, H1, Z2, H2, Z3, H3."""
+        return [_ptr(t) for zh in zip(self.Z, self.H) for t in zh]
 
 
 class SNRScreen(object):
@@ -172,10 +173,6 @@ class SNRScreen(object):
         self.y_scale = float(ls.std()) or 1.0
 
     # ----------------------------------------------------- forward/back
-    def _gemm(self, M, Nn, K, A, sam, sak, B, sbk, sbn, C, ldc, beta=0.0, split=1):
-        call('gwf_gemm_bf16', int(M), int(Nn), int(K), 1.0, _ptr(A), int(sam), int(sak), _ptr(B), int(sbk), int(sbn),
-             float(beta), _ptr(C), int(ldc), int(split), _stream())
-
     def forward_train(self, X, bt=None):
         """Standardised prediction y (B,) keeping the activations for backward."""
         B = X.shape[0]
@@ -183,36 +180,13 @@ class SNRScreen(object):
             if self._batch is None or self._batch.B != B:
                 self._batch = _Batch(B)
             bt = self._batch
-        s = _stream()
-        inp, k_in = X, KFEAT
-        for l in range(3):
-            W = self._view(self.theta_bf, 'W%d' % (l + 1))
-            self._gemm(B, HID, k_in, inp, k_in, 1, W, 1, k_in, bt.C, HID)
-            call('gwf_bias_silu', _ptr(bt.C), _ptr(self._view(self.theta, 'b%d' % (l + 1))), B, HID, _ptr(bt.Z[l]),
-                 _ptr(bt.H[l]), s)
-            inp, k_in = bt.H[l], HID
-        call('gwf_head_forward', _ptr(bt.H[2]), _ptr(self._view(self.theta, 'w4')), _ptr(self._view(self.theta, 'b4')),
-             B, _ptr(bt.y), s)
+        call('gwf_mlp_forward', _ptr(X), _ptr(self.theta_bf), _ptr(self.theta), B, *bt.acts(), _ptr(bt.y), _stream())
         return bt.y, bt
 
     def backward(self, X, bt, g):
         """Gradient of sum(g * y) into self.grad (overwritten)."""
-        B = X.shape[0]
-        s = _stream()
-        split = max(1, min(64, B // 256))
-        call('gwf_head_backward', _ptr(bt.H[2]), _ptr(self._view(self.theta, 'w4')), _ptr(g), B, _ptr(bt.dH),
-             _ptr(self._view(self.grad, 'w4')), _ptr(self._view(self.grad, 'b4')), s)
-        for l in (2, 1, 0):
-            call('gwf_silu_backward', _ptr(bt.dH), _ptr(bt.Z[l]), B * HID, _ptr(bt.dZ), _ptr(bt.dZb), s)
-            call('gwf_colsum', _ptr(bt.dZ), None, None, B, HID, _ptr(self._view(self.grad, 'b%d' % (l + 1))), 0, s)
-            inp, k_in = (bt.H[l - 1], HID) if l > 0 else (X, KFEAT)
-            # dW (out, in) = dZ^T H_prev
-            self._gemm(HID, k_in, B, bt.dZb, 1, HID, inp, k_in, 1, self._view(self.grad, 'W%d' % (l + 1)), k_in,
-                       split=split)
-            if l > 0:
-                # dH_prev (B, in) = dZ W
-                W = self._view(self.theta_bf, 'W%d' % (l + 1))
-                self._gemm(B, HID, HID, bt.dZb, HID, 1, W, HID, 1, bt.dH, HID)
+        call('gwf_mlp_backward', _ptr(X), _ptr(self.theta_bf), _ptr(self.theta), _ptr(g), X.shape[0], *bt.acts(),
+             _ptr(self.grad), _ptr(bt.ws), bt.ws.numel(), _stream())
 
     def adam_step(self, lr, beta1=0.9, beta2=0.999, eps=1e-8):
         self.step += 1

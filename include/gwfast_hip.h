@@ -338,6 +338,22 @@ int gwf_head_forward(const void* H, const float* w, const float* b, int64_t M, f
 int gwf_head_backward(const void* H, const float* w, const float* g, int64_t M, float* dH_out, float* dw_out,
                       float* db_out, void* stream);
 
+/* The whole network's training passes.  Parameters and gradient are flat:
+ * W1 (256, 16), W2, W3 (256, 256), b1, b2, b3, w4 (256 each), b4 (1);
+ * theta fp32, theta_bf16 the bf16 copy of the weights (16-byte aligned both).
+ * forward: X (B, 16) bf16 standardised features; keeps Z_l (B, 256) fp32 and
+ * H_l = bf16(SiLU(Z_l)) (B, 256) of the three hidden layers (16-byte aligned),
+ * y (B) = the network's output.
+ * backward: grad_out (136193) = gradient of sum(g y), from the forward's
+ * activations; workspace of gwf_mlp_backward_workspace_bytes(B) bytes (16-byte
+ * aligned).  Equal inputs give equal gradients, bit for bit. */
+int gwf_mlp_forward(const void* X, const void* theta_bf16, const float* theta, int64_t B, float* Z1, void* H1, float* Z2,
+                    void* H2, float* Z3, void* H3, float* y, void* stream);
+size_t gwf_mlp_backward_workspace_bytes(int64_t B);
+int gwf_mlp_backward(const void* X, const void* theta_bf16, const float* theta, const float* g, int64_t B,
+                     const float* Z1, const void* H1, const float* Z2, const void* H2, const float* Z3, const void* H3,
+                     float* grad_out, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Mean squared error: g = 2 (y - t) / n and *loss_accum += mean((y - t)^2). */
 int gwf_mse_grad(const float* y, const float* t, int64_t n, float* g_out, float* loss_accum, void* stream);
 

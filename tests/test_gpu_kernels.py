@@ -57,3 +57,69 @@ def test_block_products_against_single_arm_sums(P, res):
     for a in range(5):
         assert norm_err(arms[a], one[a]) < 1e-11
     assert norm_err(total, one.sum(axis=0)) < 1e-11
+
+
+@pytest.mark.parametrize('B', [1, 15, 17, 300, 513, 4097])
+def test_network_passes_against_their_building_blocks(B):
+    """The fused training passes at the edges of their 16-row workgroups and
+    512-row ranges: y, Z and H bit for bit those of gwf_gemm_bf16,
+    gwf_bias_silu and gwf_head_forward (same products in the same order);
+    gradients against 64-bit sums of the building blocks' bf16 dZ and H, within
+    B roundings of 2^-24 of the sum of moduli."""
+    import ctypes
+    import torch
+    from gwfast_amd import _engine as E, _native as N, screen
+    sc = screen.SNRScreen(seed=2)
+    rng = np.random.default_rng(B)
+    theta = sc.params()
+    theta[screen.OFFSETS['b1'][0]:] = rng.normal(0., 0.2, screen.N_PARAMS - screen.OFFSETS['b1'][0])
+    sc.set_params(theta)
+    x = rng.normal(0., 1., (B, screen.KFEAT))
+    x[:, screen.NFEAT:] = 0.
+    X = torch.as_tensor(x, dtype=torch.float32).to(torch.bfloat16).cuda()
+    g = torch.as_tensor(rng.normal(0., 1., B), dtype=torch.float32).cuda()
+    y, bt = sc.forward_train(X)
+    sc.backward(X, bt, g)
+    grad = sc.grad.cpu().numpy().astype(np.float64)
+    sc.backward(X, bt, g)
+    assert np.array_equal(grad, sc.grad.cpu().numpy())
+
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    v = lambda flat, name: p(sc._view(flat, name))
+    s, HID = N.stream_ptr(), screen.HID
+    new = lambda *shape: torch.empty(shape, dtype=torch.float32, device='cuda')
+    newb = lambda: torch.empty((B, HID), dtype=torch.bfloat16, device='cuda')
+    Z, H, inp, k = [], [], X, screen.KFEAT
+    for l in '123':
+        C, z, h = new(B, HID), new(B, HID), newb()
+        E.call('gwf_gemm_bf16', B, HID, k, 1.0, p(inp), k, 1, v(sc.theta_bf, 'W' + l), 1, k, 0.0, p(C), HID, 1, s)
+        E.call('gwf_bias_silu', p(C), v(sc.theta, 'b' + l), B, HID, p(z), p(h), s)
+        Z.append(z)
+        H.append(h)
+        inp, k = h, HID
+    yr = new(B)
+    E.call('gwf_head_forward', p(H[2]), v(sc.theta, 'w4'), v(sc.theta, 'b4'), B, p(yr), s)
+    assert torch.equal(y, yr)
+    for l in range(3):
+        assert torch.equal(bt.Z[l], Z[l]) and torch.equal(bt.H[l].view(torch.int16), H[l].view(torch.int16))
+
+    def check(name, ref, moduli):
+        o, n, shape = screen.OFFSETS[name]
+        d = np.abs(grad[o:o + n].reshape(shape) - ref)
+        assert np.all(d <= B * 2. ** -24 * moduli + 1e-30), (name, float(np.max(d)))
+
+    f64 = lambda t: t.to(torch.float64).cpu().numpy()
+    g64, h3 = f64(g), f64(H[2])
+    check('b4', g64.sum(), np.abs(g64).sum())
+    check('w4', g64 @ h3, np.abs(g64) @ np.abs(h3))
+    dH = g[:, None] * sc._view(sc.theta, 'w4')[None, :]
+    for l in (2, 1, 0):
+        dZ, dZb = new(B, HID), newb()
+        E.call('gwf_silu_backward', p(dH), p(Z[l]), B * HID, p(dZ), p(dZb), s)
+        dz, dzb, hp = f64(dZ), f64(dZb), f64(H[l - 1] if l else X)
+        check('b%d' % (l + 1), dz.sum(0), np.abs(dz).sum(0))
+        check('W%d' % (l + 1), dzb.T @ hp, np.abs(dzb).T @ np.abs(hp))
+        if l:
+            dH = new(B, HID)
+            E.call('gwf_gemm_bf16', B, HID, HID, 1.0, p(dZb), HID, 1, v(sc.theta_bf, 'W%d' % (l + 1)), HID, 1, 0.0,
+                   p(dH), HID, 1, s)
