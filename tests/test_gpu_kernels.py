@@ -123,3 +123,22 @@ def test_network_passes_against_their_building_blocks(B):
             dH = new(B, HID)
             E.call('gwf_gemm_bf16', B, HID, HID, 1.0, p(dZb), HID, 1, v(sc.theta_bf, 'W%d' % (l + 1)), HID, 1, 0.0,
                    p(dH), HID, 1, s)
+
+
+@pytest.mark.parametrize('n', [1, 127, 129, 300])
+def test_screen_is_the_same_for_every_batch_and_keeps_nan(n):
+    """An event's prediction does not depend on the batch it is in (the
+    128-event blocks' edges), and an event without a finite feature predicts
+    NaN and is recomputed (class 1)."""
+    import torch
+    from gwfast_amd import _engine as E, screen
+    rows = E.to_dev(E.param_rows(catalog.draw_bbh(1000, seed=9), False))
+    sc = screen.SNRScreen(seed=3)
+    sc.fit_normalisation(rows, torch.zeros(1000, dtype=torch.float64))
+    few = rows[:, :n].contiguous()
+    assert torch.equal(sc.predict_log_snr(few), sc.predict_log_snr(rows)[:n])
+    for value in (float('nan'), float('inf'), 0.):
+        few[2, n - 1] = value
+        ls = sc.predict_log_snr(few)
+        assert bool(torch.isnan(ls[n - 1])) and bool(torch.isfinite(ls[:n - 1]).all())
+        assert int(sc.classify(few)[n - 1]) == 1
