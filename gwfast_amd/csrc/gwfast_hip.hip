@@ -50,6 +50,89 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Wave sums of N values a lane, each of them bit for bit wave_sum's, spread
+// over the lanes: at the step of lane bit 32, 16, .. 1 half the lanes keep
+// the first half of the values and send the other, so N = 66 takes 69
+// shuffles of a double where 66 wave_sums take 396, and the stores that follow
+// two per lane instead of 66 of one lane each.  At the end of every event, the
+// longer form took some 8 % of the Fisher kernels' time (10^4 IMRPhenomD
+// events x 2000 points 1.46 -> 1.30 ms, 2 x 10^4 ragged tidal TaylorF2 events
+// 8.05 -> 7.44 ms, outputs bit for bit the same).  Lane l holds, in v[r], the
+// sum of value index(l, r) (N: none; a value left over at an odd split ends in
+// several lanes, index gives it to one).
+template <int N>
+struct WaveSums {
+  // values kept before step s: N halved s times, rounded up (in closed form: as
+  // a recursion it became real calls on a stack of unknown size)
+  static constexpr int m(int s) { return (N + (1 << s) - 1) >> s; }
+  static constexpr int R = m(6);
+  double v[N];
+  template <int S>
+  __device__ __forceinline__ void step(int lane) {
+    if constexpr (S < 6) {
+      constexpr int off = 32 >> S, M = m(S), H = m(S + 1);
+      const bool up = (lane & off) != 0;
+#pragma unroll
+      for (int j = 0; j < H; ++j) {
+        if (j + H < M) {
+          const double keep = up ? v[j + H] : v[j], send = up ? v[j] : v[j + H];
+          v[j] = keep + __shfl_xor(send, off, 64);
+        } else {
+          v[j] += __shfl_xor(v[j], off, 64);
+        }
+        // a few in flight: all at once, the values sent and kept would spill
+        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      step<S + 1>(lane);
+    }
+  }
+  __device__ __forceinline__ WaveSums(const double* x, int lane) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = x[i];
+    step<0>(lane);
+  }
+  __device__ __forceinline__ static int index(int lane, int r) {
+    int i = r;
+    bool first = true;
+#pragma unroll
+    for (int s = 5; s >= 0; --s) {
+      if (lane & (32 >> s)) {
+        if (i + m(s + 1) < m(s))
+          i += m(s + 1);
+        else
+          first = false;
+      }
+    }
+    return first ? i : N;
+  }
+  // the sum of value i (any lane's), in every lane that asks
+  __device__ __forceinline__ double of(int i) const {
+    int lane = 0;
+#pragma unroll
+    for (int s = 0; s < 6; ++s) {
+      if (i >= m(s + 1)) {
+        i -= m(s + 1);
+        lane |= 32 >> s;
+      }
+    }
+    double t = __shfl(v[0], lane, 64);
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+      const double u = __shfl(v[r], lane, 64);
+      t = i == r ? u : t;
+    }
+    return t;
+  }
+};
+
+// row and column of element i of a packed upper triangle of n rows
+__device__ __forceinline__ void unpack_upper(int i, int n, int* row, int* col) {
+  int a = 0, c = i;
+  while (c >= n - a) c -= n - a++;
+  *row = a;
+  *col = a + c;
+}
+
 __device__ __forceinline__ int64_t wave_event() {
   const int wave = threadIdx.x >> 6;
   const int64_t e = (int64_t)blockIdx.x * WAVES_PER_BLOCK + wave;
@@ -121,18 +204,16 @@ __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const d
 // Wave-reduces the packed Gram and writes the symmetric (P, P, n_ev) output.
 template <int P>
 __device__ __forceinline__ void store_packed(const double* G, double* __restrict__ F, int64_t n_ev, int64_t e, int lane) {
-  int k = 0;
+  constexpr int NG = P * (P + 1) / 2;
+  const WaveSums<NG> sums(G, lane);
 #pragma unroll
-  for (int a = 0; a < P; ++a) {
-#pragma unroll
-    for (int b = a; b < P; ++b) {
-      const double s = wave_sum(G[k]);
-      if (lane == (k & 63)) {
-        F[(int64_t)(a * P + b) * n_ev + e] = s;
-        if (a != b) F[(int64_t)(b * P + a) * n_ev + e] = s;
-      }
-      ++k;
-    }
+  for (int r = 0; r < WaveSums<NG>::R; ++r) {
+    const int i = WaveSums<NG>::index(lane, r);
+    if (i >= NG) continue;
+    int a, b;
+    unpack_upper(i, P, &a, &b);
+    F[(int64_t)(a * P + b) * n_ev + e] = sums.v[r];
+    if (a != b) F[(int64_t)(b * P + a) * n_ev + e] = sums.v[r];
   }
 }
 
@@ -537,21 +618,19 @@ __device__ __forceinline__ void store_pure_mx(const double* G, const double* acc
     F[(int64_t)(a * P + b) * n_ev + e] = v;
     if (a != b) F[(int64_t)(b * P + a) * n_ev + e] = v;
   };
-  int k = 0;
+  constexpr int NG = 28 + NPU * (NPU + 1) / 2;
+  const WaveSums<NG> sums(G, lane);
 #pragma unroll
-  for (int a = 0; a < 7; ++a)
-#pragma unroll
-    for (int b = a; b < 7; ++b, ++k) {
-      const double s = wave_sum(G[pk<7>(a, b)]);
-      if (lane == (k & 63)) put(NP[a], NP[b], s);
-    }
-#pragma unroll
-  for (int p = 0; p < NPU; ++p)
-#pragma unroll
-    for (int q = p; q < NPU; ++q, ++k) {
-      const double s = wave_sum(G[28 + pk<NPU>(p, q)]);
-      if (lane == (k & 63)) put(PU(p), PU(q), s);
-    }
+  for (int r = 0; r < WaveSums<NG>::R; ++r) {
+    const int i = WaveSums<NG>::index(lane, r);
+    if (i >= NG) continue;
+    int a, b;
+    unpack_upper(i < 28 ? i : i - 28, i < 28 ? 7 : NPU, &a, &b);
+    if (i < 28)
+      put(a < 2 ? a : a + 1, b < 2 ? b : b + 1, sums.v[r]);
+    else
+      put(PU(a), PU(b), sums.v[r]);
+  }
 #pragma unroll
   for (int g = 0; g < 2; ++g)
 #pragma unroll
@@ -750,44 +829,35 @@ template <int P>
 __device__ __forceinline__ void store_semi_vx(const double* G, const double* acc, double* __restrict__ F, int64_t n_ev,
                                               int64_t e, int lane) {
   constexpr int NF = P - 4, NFF = NF * (NF + 1) / 2;
-  constexpr int SK[4] = {3, 4, 5, 6};
   auto put = [&](int a, int b, double v) {
     F[(int64_t)(a * P + b) * n_ev + e] = v;
     if (a != b) F[(int64_t)(b * P + a) * n_ev + e] = v;
   };
-  int q = 0;
+  constexpr int NG = NFF + 22;
+  const WaveSums<NG> sums(G, lane);
 #pragma unroll
-  for (int j = 0; j < NF; ++j)
-#pragma unroll
-    for (int l = j; l < NF; ++l, ++q) {
-      const double s = wave_sum(G[q]);
-      if (lane == (q & 63)) put(semi_row<P>(j), semi_row<P>(l), s);
-    }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = a; b < 4; ++b) {
-      const double s = wave_sum(G[NFF + 12 + pk<4>(a, b)]);
-      if (lane == ((NFF + pk<4>(a, b)) & 63)) put(SK[a], SK[b], s);
-    }
+  for (int r = 0; r < WaveSums<NG>::R; ++r) {
+    const int i = WaveSums<NG>::index(lane, r);
+    if (i >= NG || (i >= NFF && i < NFF + 12)) continue;
+    int a, b;
+    unpack_upper(i < NFF ? i : i - NFF - 12, i < NFF ? NF : 4, &a, &b);
+    if (i < NFF)
+      put(semi_row<P>(a), semi_row<P>(b), sums.v[r]);
+    else
+      put(3 + a, 3 + b, sums.v[r]);
+  }
   // sky x factored: the matrix-core part (element (j, k) in lane k + 16 (j % 4)
   // of group j / 4) plus, for the rows with s_j != 0, the wave sum of s_j Tv_k
-  double st[12];
-#pragma unroll
-  for (int i = 0; i < 12; ++i) st[i] = wave_sum(G[NFF + i]);
   const int k = lane & 3;
 #pragma unroll
   for (int r = 0; r < (NF + 3) / 4; ++r) {
     const int j = (lane >> 4) + 4 * r;
     double v = block_sum(acc[r]);
-    if (j < NF && (lane & 12) == 0) {
-#pragma unroll
-      for (int jj = 0; jj < 3; ++jj)
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-          if (j == jj && k == kk) v += st[4 * jj + kk];
-      put(semi_row<P>(j), SK[k], v);
+    if (r == 0) {
+      const double st = sums.of(NFF + min(4 * j + k, 11));
+      if (j < 3) v += st;
     }
+    if (j < NF && (lane & 12) == 0) put(semi_row<P>(j), 3 + k, v);
   }
 }
 
@@ -831,6 +901,14 @@ __device__ __forceinline__ void store_mx(const double* acc, double* __restrict__
 #ifndef GWF_PQ_MFMA_MIN_P
 #define GWF_PQ_MFMA_MIN_P 12
 #endif
+
+// (a consumer's sums are cleared as they are stored, not at the next event's
+// first chunk, so that the compiler need not keep them through the store)
+template <int N>
+__device__ __forceinline__ void set_zero(double (&x)[N]) {
+#pragma unroll
+  for (int q = 0; q < N; ++q) x[q] = 0.0;
+}
 
 // Consumer side of a pair: waits for each item in turn, runs item(e, t,
 // res, chunk) on it, releases its buffer and, after the last chunk of event
@@ -967,35 +1045,35 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
     if (SEMI_VX && !net.mixed_motion) {
       constexpr int NF = P - 4, NG = NF * (NF + 1) / 2 + 12 + 10;
       double G[NG], acc[(NF + 3) / 4];
+      set_zero(G);
+      set_zero(acc);
       pq_consumer<NB>(&cnt[slot][0], &cnt[slot][1], head[slot], buf[slot], counter, net.spin_limit, lane,
                       [&](int e, int t, int res, const double* chunk) {
-                        if (t == 0) {
-#pragma unroll
-                          for (int q = 0; q < NG; ++q) G[q] = 0.0;
-#pragma unroll
-                          for (int q = 0; q < (NF + 3) / 4; ++q) acc[q] = 0.0;
-                        }
                         pc_consume_semi_vx<MODEL, NT, P>(net, rec + (int64_t)e * REC_DOUBLES, t * 64, res, lane,
                                                          chunk, X, G, acc);
                       },
-                      [&](int e) { store_semi_vx<P>(G, acc, F, n_ev, e, lane); });
+                      [&](int e) {
+                        store_semi_vx<P>(G, acc, F, n_ev, e, lane);
+                        set_zero(G);
+                        set_zero(acc);
+                      });
       return;
     }
 #endif
     constexpr int NPU = P - 7, NG = 28 + NPU * (NPU + 1) / 2;
     double G[NG], acc[4];
+    set_zero(G);
+    set_zero(acc);
     pq_consumer<NB>(&cnt[slot][0], &cnt[slot][1], head[slot], buf[slot], counter, net.spin_limit, lane,
                     [&](int e, int t, int res, const double* chunk) {
-                      if (t == 0) {
-#pragma unroll
-                        for (int q = 0; q < NG; ++q) G[q] = 0.0;
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) acc[q] = 0.0;
-                      }
                       pc_consume_pure_mx<MODEL, NT, P>(net, rec + (int64_t)e * REC_DOUBLES, t * 64, res, lane, chunk,
                                                        X, G, acc);
                     },
-                    [&](int e) { store_pure_mx<P>(G, acc, F, n_ev, e, lane); });
+                    [&](int e) {
+                      store_pure_mx<P>(G, acc, F, n_ev, e, lane);
+                      set_zero(G);
+                      set_zero(acc);
+                    });
   } else if constexpr (MX) {  // Gram on the matrix cores
     double* X = xt[slot];
     for (int q = lane; q < PQ_TILE; q += 64) X[q] = 0.0;  // padding columns stay zero
@@ -1003,33 +1081,30 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
       if (!net.mixed_motion) {
         constexpr int NF = P - 4, NG = NF * (NF + 1) / 2 + 12 + 10;
         double G[NG], acc1[(NF + 3) / 4];
+        set_zero(G);
+        set_zero(acc1);
         uint32_t mask = 0u;
         pq_consumer<NB>(&cnt[slot][0], &cnt[slot][1], head[slot], buf[slot], counter, net.spin_limit, lane,
                         [&](int e, int t, int res, const double* chunk) {
-                          if (t == 0) {
-#pragma unroll
-                            for (int q = 0; q < NG; ++q) G[q] = 0.0;
-#pragma unroll
-                            for (int q = 0; q < (NF + 3) / 4; ++q) acc1[q] = 0.0;
-                            mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)arm_mask[e]);
-                          }
+                          if (t == 0) mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)arm_mask[e]);
                           pc_consume_semi_vx<MODEL, NT, P, true>(net, rec + (int64_t)e * REC_DOUBLES, t * 64, res,
                                                                  lane, chunk, X, G, acc1, mask);
                         },
-                        [&](int e) { store_semi_vx<P>(G, acc1, F, n_ev, e, lane); });
+                        [&](int e) {
+                          store_semi_vx<P>(G, acc1, F, n_ev, e, lane);
+                          set_zero(G);
+                          set_zero(acc1);
+                        });
         return;
       }
     }
     constexpr int NB2 = GramBlocks<P>::ACCS, NA = ARMS ? PQ_ARMS_MAX * NB2 : NB2;  // ARMS: a set per physical arm
     double acc[NA];
+    set_zero(acc);
     uint32_t mask = 0u;
     pq_consumer<NB>(&cnt[slot][0], &cnt[slot][1], head[slot], buf[slot], counter, net.spin_limit, lane,
                     [&](int e, int t, int res, const double* chunk) {
-                      if (t == 0) {
-#pragma unroll
-                        for (int q = 0; q < NA; ++q) acc[q] = 0.0;
-                        if (MASKED) mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)arm_mask[e]);
-                      }
+                      if (MASKED && t == 0) mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)arm_mask[e]);
                       pc_consume_mx<MODEL, NT, P, MODE>(net, rec + (int64_t)e * REC_DOUBLES, t * 64, res, lane, chunk,
                                                         X, acc, mask);
                     },
@@ -1042,10 +1117,12 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
                       } else {
                         store_mx<P>(acc, F, n_ev, e, lane);
                       }
+                      set_zero(acc);
                     });
   } else {  // Gram on the VALU, packed upper triangle per lane
     constexpr int NG = P * (P + 1) / 2;
     double G[NG];
+    set_zero(G);
     uint32_t mask = 0u;
     // KIND 0: no row factored, 1: the pure rows, 2: the pure rows and the
     // Mc, eta, tcoal rows (pc_consume_semi).  Chosen once per wave, so that
@@ -1054,11 +1131,7 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
       constexpr int KIND = decltype(kind)::value;
       pq_consumer<NB>(&cnt[slot][0], &cnt[slot][1], head[slot], buf[slot], counter, net.spin_limit, lane,
                       [&](int e, int t, int res, const double* chunk) {
-                        if (t == 0) {
-#pragma unroll
-                          for (int q = 0; q < NG; ++q) G[q] = 0.0;
-                          if (MASKED) mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)arm_mask[e]);
-                        }
+                        if (MASKED && t == 0) mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)arm_mask[e]);
                         const double* r = rec + (int64_t)e * REC_DOUBLES;
                         if constexpr (KIND == 2)
                           pc_consume_semi<MODEL, NT, MASKED>(net, r, t * 64, res, lane, chunk, G, mask);
@@ -1067,7 +1140,10 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
                         else
                           pc_consume<MODEL, NT, P, MASKED>(net, r, t * 64, res, lane, chunk, G, mask);
                       },
-                      [&](int e) { store_packed<P>(G, F, n_ev, e, lane); });
+                      [&](int e) {
+                        store_packed<P>(G, F, n_ev, e, lane);
+                        set_zero(G);
+                      });
     };
 #ifdef GWF_NO_PURE_ROWS
     consume(std::integral_constant<int, 0>{});
