@@ -139,6 +139,20 @@ __device__ __forceinline__ int64_t wave_event() {
   return (int64_t)__builtin_amdgcn_readfirstlane((int)e);
 }
 
+// Block b of n handed to the XCDs in turn (b % 8), renumbered so that an XCD's
+// blocks are neighbours: rows of a (points, events) array, read a few events
+// at a time, are then shared in that XCD's L2 instead of being fetched by all
+// eight.  Blocks past the last full eight keep their number.
+__device__ __forceinline__ int64_t near_block(int64_t b, int64_t n) {
+  const int64_t per = n / 8;
+  return b < 8 * per ? (b % 8) * per + b / 8 : b;
+}
+__device__ __forceinline__ int64_t near_event() {
+  const int wave = threadIdx.x >> 6;
+  const int64_t e = near_block(blockIdx.x, gridDim.x) * WAVES_PER_BLOCK + wave;
+  return (int64_t)__builtin_amdgcn_readfirstlane((int)e);
+}
+
 // ------------------------------------------------------------------ kernels
 // Minimum of each event's column of a caller's grid f (nf, n_ev), into the
 // event's record at REC_F0 (a site slot that records with a caller's grid,
@@ -1250,10 +1264,13 @@ __global__ __launch_bounds__(256) void k_strain(gwf_waveform w, NetK net, const 
                                                 int armi, const double* __restrict__ f, int64_t nf,
                                                 double* __restrict__ h, double* __restrict__ J,
                                                 double* __restrict__ comp) {
-  const int64_t e = wave_event();
+  const int64_t e = near_event();
   if (e >= n_ev) return;
   const int lane = threadIdx.x & 63;
-  strain_event<MODEL, NT, P>(w, net, rec + e * (int64_t)REC_DOUBLES, armi, f + e, n_ev, nf, lane, 64,
+  // waves of grid row y take chunks y, y + gridDim.y, ... of the event's points
+  // (500 IMRPhenomD events x 2000 points: one wave each 137 us, sixteen 63)
+  strain_event<MODEL, NT, P>(w, net, rec + e * (int64_t)REC_DOUBLES, armi, f + e, n_ev, nf,
+                             lane + 64 * (int)blockIdx.y, 64 * (int)gridDim.y,
                              h ? h + 2 * e : nullptr, 2 * n_ev, J ? J + 2 * e * nf : nullptr, 2 * n_ev * nf,
                              comp ? comp + e : nullptr, n_ev, nf * n_ev);
 }
@@ -1346,46 +1363,74 @@ __global__ void k_fcut(gwf_waveform w, const double* __restrict__ par, int64_t l
   out[e] = fcut_eff(fc, fmax);
 }
 
-// Plain Gram over materialised derivatives (one wave per event).
+// Plain Gram over materialised derivatives, bound by the read of J (16 P
+// bytes per point).  wpe waves per event (1 or WAVES_PER_BLOCK) take its
+// chunks of 64 points in turn, their sums added through LDS: with one wave
+// per event, 2000 events leave most of the loads the chip can hold in flight
+// unused.  f and S are read across events, so a block's neighbours run on its
+// XCD (near_block), and a lane takes its neighbours' f by shuffles.  2000
+// events x 1000 points, P = 11: 141 -> 117 us, 3.0 TB/s (with four waves'
+// sums by wave_sum 204 us, bound by the LDS of its shuffles).
 template <int P>
 __global__ __launch_bounds__(256) void k_gram(const double* __restrict__ J, const double* __restrict__ f,
-                                              const double* __restrict__ S, int64_t n_ev, int64_t nf, int accumulate,
-                                              double* __restrict__ F) {
-  const int64_t e = wave_event();
-  if (e >= n_ev) return;
-  const int lane = threadIdx.x & 63;
+                                              const double* __restrict__ S, int64_t n_ev, int64_t nf, int wpe,
+                                              int accumulate, double* __restrict__ F) {
   constexpr int NG = P * (P + 1) / 2;
-  double G[NG];
+  __shared__ double part[WAVES_PER_BLOCK][NG];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t b = near_block(blockIdx.x, gridDim.x);
+  const int64_t e = (int64_t)__builtin_amdgcn_readfirstlane((int)(wpe == 1 ? b * WAVES_PER_BLOCK + wave : b));
+  if (e < n_ev) {
+    double G[NG];
 #pragma unroll
-  for (int k = 0; k < NG; ++k) G[k] = 0.0;
-  const int64_t js = 2 * n_ev * nf;
-  const double* Je = J + 2 * e * nf;
-  for (int64_t i = lane; i < nf; i += 64) {
-    const double fi = f[i * n_ev + e];
-    const double fl = i > 0 ? f[(i - 1) * n_ev + e] : fi;
-    const double fr = i < nf - 1 ? f[(i + 1) * n_ev + e] : fi;
-    const double wS = 4.0 * 0.5 * (fr - fl) / S[i * n_ev + e];
-    double re[P], im[P];
+    for (int k = 0; k < NG; ++k) G[k] = 0.0;
+    const int64_t js = 2 * n_ev * nf;
+    const double* Je = J + 2 * e * nf;
+    const double* fe = f + e;
+    for (int64_t base = wpe == 1 ? 0 : 64 * wave; base < nf; base += 64 * wpe) {
+      const int64_t i = base + lane;
+      const bool live = i < nf;
+      double fi = 0.0, edge = 0.0, Si = 1.0;
+      double re[P], im[P];
+      if (live) {
+        fi = fe[i * n_ev];
+        Si = S[i * n_ev + e];
 #pragma unroll
-    for (int X = 0; X < P; ++X) {
-      re[X] = Je[X * js + 2 * i];
-      im[X] = Je[X * js + 2 * i + 1];
-    }
-    gram_update<P>(G, re, im, wS);
-  }
-  int k = 0;
-#pragma unroll
-  for (int a = 0; a < P; ++a) {
-#pragma unroll
-    for (int b = a; b < P; ++b) {
-      const double s = wave_sum(G[k]);
-      if (lane == (k & 63)) {
-        const int64_t i1 = (int64_t)(a * P + b) * n_ev + e, i2 = (int64_t)(b * P + a) * n_ev + e;
-        F[i1] = accumulate ? F[i1] + s : s;
-        if (a != b) F[i2] = accumulate ? F[i2] + s : s;
+        for (int X = 0; X < P; ++X) {
+          re[X] = Je[X * js + 2 * i];
+          im[X] = Je[X * js + 2 * i + 1];
+        }
       }
-      ++k;
+      const int64_t ie = lane == 0 ? max(i - 1, (int64_t)0) : min(i + 1, nf - 1);
+      if (live && (lane == 0 || lane == 63 || i == nf - 1)) edge = fe[ie * n_ev];
+      double fl = __shfl_up(fi, 1, 64), fr = __shfl_down(fi, 1, 64);
+      if (lane == 0) {
+        fl = edge;
+        if (i == nf - 1) fr = fi;
+      } else if (lane == 63 || i == nf - 1) {
+        fr = edge;
+      }
+      if (!live) continue;
+      const double wS = 4.0 * 0.5 * (fr - fl) / Si;
+      gram_update<P>(G, re, im, wS);
     }
+    const WaveSums<NG> sums(G, lane);
+#pragma unroll
+    for (int r = 0; r < WaveSums<NG>::R; ++r) {
+      const int k = WaveSums<NG>::index(lane, r);
+      if (k < NG) part[wave][k] = sums.v[r];
+    }
+  }
+  __syncthreads();
+  if (e >= n_ev) return;
+  for (int k = wpe == 1 ? lane : (int)threadIdx.x; k < NG; k += 64 * wpe) {
+    double s = part[wpe == 1 ? wave : 0][k];
+    for (int w = 1; w < wpe; ++w) s += part[w][k];
+    int a, c;
+    unpack_upper(k, P, &a, &c);
+    const int64_t i1 = (int64_t)(a * P + c) * n_ev + e, i2 = (int64_t)(c * P + a) * n_ev + e;
+    F[i1] = accumulate ? F[i1] + s : s;
+    if (a != c) F[i2] = accumulate ? F[i2] + s : s;
   }
 }
 
@@ -1465,19 +1510,62 @@ __global__ __launch_bounds__(256) void k_gram_split(const double* __restrict__ J
   }
 }
 
-// VJP of the strain: one wave per (parameter, event) pair.
-__global__ __launch_bounds__(256) void k_vjp(const double* __restrict__ J, const double* __restrict__ gh, int P,
-                                             int64_t n_ev, int64_t nf, double tc_scale, double* __restrict__ g) {
-  const int64_t pe = wave_event();
-  if (pe >= (int64_t)P * n_ev) return;
-  const int lane = threadIdx.x & 63;
-  const int64_t p = pe / n_ev, e = pe % n_ev;
-  const double* Jr = J + 2 * (p * n_ev + e) * nf;
-  double acc = 0.0;
-  for (int64_t i = lane; i < nf; i += 64)
-    acc += gh[2 * (i * n_ev + e)] * Jr[2 * i] + gh[2 * (i * n_ev + e) + 1] * Jr[2 * i + 1];
-  acc = wave_sum(acc);
-  if (lane == 0) g[p * n_ev + e] = (p == 7) ? acc * tc_scale : acc;
+// VJP of the strain, bound by the read of J: a block per event, whose lanes
+// take a point and all PB parameters of a pass at a time (gh, read across
+// events, once per pass instead of once per parameter, and shared with the
+// neighbouring blocks in the XCD's L2), sums added through LDS in wave order.
+// 500 events x 2000 points, P = 11: 66 -> 31 us, 6 TB/s; a wave per parameter
+// and event read gh eleven times, a line of it per lane.
+template <int PB>
+__device__ __forceinline__ void vjp_pass(const double* __restrict__ J, const double* __restrict__ gh, int p0,
+                                         int64_t n_ev, int64_t nf, int64_t e, double tc_scale, double* __restrict__ g,
+                                         double (*part)[16]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const double* Je = J + 2 * ((int64_t)p0 * n_ev + e) * nf;
+  const int64_t js = 2 * n_ev * nf;
+  double acc[PB];
+#pragma unroll
+  for (int p = 0; p < PB; ++p) acc[p] = 0.0;
+  for (int64_t i = threadIdx.x; i < nf; i += BLOCK) {
+    const double gr = gh[2 * (i * n_ev + e)], gi = gh[2 * (i * n_ev + e) + 1];
+    double re[PB], im[PB];
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+      re[p] = Je[p * js + 2 * i];
+      im[p] = Je[p * js + 2 * i + 1];
+    }
+#pragma unroll
+    for (int p = 0; p < PB; ++p) acc[p] += gr * re[p] + gi * im[p];
+  }
+#pragma unroll
+  for (int p = 0; p < PB; ++p) {
+    const double s = wave_sum(acc[p]);
+    if (lane == 0) part[wave][p] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < PB) {
+    double s = part[0][threadIdx.x];
+    for (int w = 1; w < WAVES_PER_BLOCK; ++w) s += part[w][threadIdx.x];
+    const int p = p0 + threadIdx.x;
+    g[p * n_ev + e] = p == 7 ? s * tc_scale : s;
+  }
+  __syncthreads();
+}
+// PT > 0: all P = PT parameters in one pass (the models' 11 to 14)
+template <int PT>
+__global__ __launch_bounds__(BLOCK) void k_vjp(const double* __restrict__ J, const double* __restrict__ gh, int P,
+                                               int64_t n_ev, int64_t nf, double tc_scale, double* __restrict__ g) {
+  __shared__ double part[WAVES_PER_BLOCK][16];
+  for (int64_t b = blockIdx.x; b < n_ev; b += gridDim.x) {
+    const int64_t e = near_block(b, n_ev);
+    if constexpr (PT > 0) {
+      vjp_pass<PT>(J, gh, 0, n_ev, nf, e, tc_scale, g, part);
+    } else {
+      int p = 0;
+      for (; p + 4 <= P; p += 4) vjp_pass<4>(J, gh, p, n_ev, nf, e, tc_scale, g, part);
+      for (; p < P; ++p) vjp_pass<1>(J, gh, p, n_ev, nf, e, tc_scale, g, part);
+    }
+  }
 }
 
 // ------------------------------------------- covariance (one wave per event)
@@ -2989,6 +3077,7 @@ int gwf_fisher_ragged(const gwf_waveform* wf, const gwf_detector* dets, int32_t 
   return hip_check(hipGetLastError(), "gwf_fisher_ragged launch");
 }
 
+constexpr int64_t STRAIN_WAVES = 8192;
 static int strain_impl(const gwf_waveform* wf, const gwf_detector* det, int32_t arm, const double* params, int64_t ld,
                        int64_t n_ev, const double* f, int64_t n_f, double* h_out, double* J_out, double* comp_out,
                        void* workspace, size_t ws_bytes, void* stream) {
@@ -3003,7 +3092,10 @@ static int strain_impl(const gwf_waveform* wf, const gwf_detector* det, int32_t 
   hipStream_t st = (hipStream_t)stream;
   rc = launch_setup(wf, net, params, ld, n_ev, f, n_f, (double*)workspace, st);
   if (rc) return rc;
-  const dim3 grid((unsigned)((n_ev + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK)), block(BLOCK);
+  // each event's points over as many waves as fill the chip eight to a SIMD,
+  // a chunk of 64 points each at least
+  const int64_t rows = std::max<int64_t>(1, std::min<int64_t>((n_f + 63) / 64, STRAIN_WAVES / n_ev));
+  const dim3 grid((unsigned)((n_ev + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK), (unsigned)rows), block(BLOCK);
   const double* rec = (const double*)workspace;
   if (wf->model == GWF_MODEL_IMRPHENOMD)
     hipLaunchKernelGGL((k_strain<GWF_MODEL_IMRPHENOMD, 4, 11>), grid, block, 0, st, *wf, net, rec, n_ev, (int)arm, f,
@@ -3045,9 +3137,20 @@ int gwf_strain_vjp(const double* J, const double* gh, int32_t P, int64_t n_ev, i
   if ((int64_t)P * n_ev == 0) return 0;
   if (!J || !gh || !g_out) return fail(-EINVAL, "NULL array");
   if ((int64_t)P * n_ev > (int64_t)0x7fffffff / WAVES_PER_BLOCK) return fail(-EINVAL, "too many events for one call");
-  const int64_t waves = (int64_t)P * n_ev;
-  hipLaunchKernelGGL(k_vjp, dim3((unsigned)((waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK)), dim3(BLOCK), 0,
-                     (hipStream_t)stream, J, gh, (int)P, n_ev, n_f, tcoal_scale, g_out);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(n_ev, 1 << 20)), dim3(BLOCK), 0, (hipStream_t)stream, J, gh, (int)P, n_ev, n_f,
+                       tcoal_scale, g_out);
+  };
+  if (P == 11)
+    go(k_vjp<11>);
+  else if (P == 12)
+    go(k_vjp<12>);
+  else if (P == 13)
+    go(k_vjp<13>);
+  else if (P == 14)
+    go(k_vjp<14>);
+  else
+    go(k_vjp<0>);
   return hip_check(hipGetLastError(), "gwf_strain_vjp launch");
 }
 
@@ -3058,16 +3161,18 @@ int gwf_gram(const double* J, const double* f, const double* S, int32_t P, int64
   if (n_ev == 0) return 0;
   if (!J || !f || !S || !fisher_out) return fail(-EINVAL, "NULL array");
   if (n_ev > (int64_t)0x7fffffff / WAVES_PER_BLOCK) return fail(-EINVAL, "too many events for one call");
-  const dim3 grid((unsigned)((n_ev + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK)), block(BLOCK);
+  // a block's waves share an event where its grid has a chunk for each of them
+  const int wpe = n_f > 64 * (WAVES_PER_BLOCK - 1) ? WAVES_PER_BLOCK : 1;
+  const dim3 grid((unsigned)(wpe == 1 ? (n_ev + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK : n_ev)), block(BLOCK);
   hipStream_t st = (hipStream_t)stream;
   if (P == 11)
-    hipLaunchKernelGGL((k_gram<11>), grid, block, 0, st, J, f, S, n_ev, n_f, (int)accumulate, fisher_out);
+    hipLaunchKernelGGL((k_gram<11>), grid, block, 0, st, J, f, S, n_ev, n_f, wpe, (int)accumulate, fisher_out);
   else if (P == 12)
-    hipLaunchKernelGGL((k_gram<12>), grid, block, 0, st, J, f, S, n_ev, n_f, (int)accumulate, fisher_out);
+    hipLaunchKernelGGL((k_gram<12>), grid, block, 0, st, J, f, S, n_ev, n_f, wpe, (int)accumulate, fisher_out);
   else if (P == 13)
-    hipLaunchKernelGGL((k_gram<13>), grid, block, 0, st, J, f, S, n_ev, n_f, (int)accumulate, fisher_out);
+    hipLaunchKernelGGL((k_gram<13>), grid, block, 0, st, J, f, S, n_ev, n_f, wpe, (int)accumulate, fisher_out);
   else
-    hipLaunchKernelGGL((k_gram<14>), grid, block, 0, st, J, f, S, n_ev, n_f, (int)accumulate, fisher_out);
+    hipLaunchKernelGGL((k_gram<14>), grid, block, 0, st, J, f, S, n_ev, n_f, wpe, (int)accumulate, fisher_out);
   return hip_check(hipGetLastError(), "gwf_gram launch");
 }
 

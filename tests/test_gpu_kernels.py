@@ -142,3 +142,62 @@ def test_screen_is_the_same_for_every_batch_and_keeps_nan(n):
         ls = sc.predict_log_snr(few)
         assert bool(torch.isnan(ls[n - 1])) and bool(torch.isfinite(ls[:n - 1]).all())
         assert int(sc.classify(few)[n - 1]) == 1
+
+
+@pytest.mark.parametrize('P', [11, 12, 13, 14])
+@pytest.mark.parametrize('n,nf', [(1, 1), (5, 63), (3, 64), (9, 192), (17, 193), (8, 257), (66, 1000)])
+def test_gram_over_an_events_waves(P, n, nf):
+    """The plain Gram, one wave or four per event, against torch in FP64: sums
+    of 2 nf products, so 4 nf 2^-52 of the sums of moduli."""
+    import torch
+    from gwfast_amd import _engine as E, signal as S
+    rng = np.random.default_rng(nf)
+    J, f = rng.standard_normal((P, n, nf, 2)), np.sort(rng.uniform(1., 9., (nf, n)), axis=0)
+    psd = rng.uniform(0.5, 2., (nf, n))
+    got = S.gram_device(E.to_dev(J), E.to_dev(f), E.to_dev(psd), P)
+    twice = S.gram_device(E.to_dev(J), E.to_dev(f), E.to_dev(psd), P, out=got.clone(), accumulate=True)
+    w = np.zeros_like(f)
+    w[1:] += 0.5 * np.diff(f, axis=0)
+    w[:-1] += 0.5 * np.diff(f, axis=0)
+    x = J * np.sqrt(4. * w / psd).T[None, :, :, None]
+    x = x.reshape(P, n, -1).transpose(1, 0, 2)
+    ref, mod = x @ x.transpose(0, 2, 1), np.abs(x) @ np.abs(x).transpose(0, 2, 1)
+    d = np.abs(got.cpu().numpy().transpose(2, 0, 1) - ref)
+    assert np.all(d <= 4 * nf * 2. ** -52 * mod + 1e-300)
+    assert torch.equal(twice, 2 * got)
+
+
+@pytest.mark.parametrize('P', [1, 3, 4, 6, 11, 12, 13, 14, 16])
+@pytest.mark.parametrize('n,nf', [(1, 1), (3, 255), (9, 256), (17, 700)])
+def test_strain_vjp_at_any_parameter_count(P, n, nf):
+    """g_p = sum_f Re(conj(gh) J_p) against numpy in FP64 (4 nf 2^-52 of the
+    sum of moduli; the tcoal row scaled)."""
+    import torch
+    from gwfast_amd import _engine as E, _native as N
+    rng = np.random.default_rng(nf)
+    J, gh = rng.standard_normal((P, n, nf, 2)), rng.standard_normal((nf, n, 2))
+    Jd, gd, g = E.to_dev(J), E.to_dev(gh), torch.empty((P, n), dtype=torch.float64, device='cuda')
+    E.call('gwf_strain_vjp', N.ptr(Jd), N.ptr(gd), P, n, nf, 86400.0, N.ptr(g), N.stream_ptr())
+    s = np.ones((P, 1))
+    s[7:8] = 86400.
+    prod = J * gh.transpose(1, 0, 2)[None]
+    d = np.abs(g.cpu().numpy() - s * prod.sum(axis=(2, 3)))
+    assert np.all(d <= 4 * nf * 2. ** -52 * s * np.abs(prod).sum(axis=(2, 3)))
+
+
+@pytest.mark.parametrize('P', [11, 13])
+@pytest.mark.parametrize('n,nf', [(1, 1), (1, 64), (3, 130), (3, 500)])
+def test_strain_split_over_an_events_points(P, n, nf):
+    """Few events, their points spread over many waves, against the same
+    events among 9000 (one wave each): bit for bit."""
+    from tests._common import NET_C0, hip_net
+    from gwfast_amd import _engine as E, signal as S
+    wf = _wf(P)
+    rows = E.to_dev(E.param_rows(_events(P, n, 6), P == 13))
+    f = E.to_dev(np.geomspace(np.full(n, 3.), np.full(n, 50.), nf))
+    sig = list(hip_net(wf, NET_C0, True).signals.values())[0]
+    k = 9000 // n
+    h, J = S.strain_device(sig, rows, f, 0)
+    hm, Jm = S.strain_device(sig, rows.repeat(1, k).contiguous(), f.repeat(1, k).contiguous(), 0)
+    assert np.array_equal(h.cpu().numpy(), hm[:, :n].cpu().numpy())
+    assert np.array_equal(J.cpu().numpy(), Jm[:, :n].cpu().numpy())
