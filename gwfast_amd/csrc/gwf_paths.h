@@ -303,6 +303,34 @@ GWF_HD void setup_waveform_split(const gwf_waveform& w, const double* par, int64
 template <int MODEL>
 GWF_HD void setup_event_consts(const NetK& net, const double* par, int64_t ld, int64_t e, double* rec);
 
+// The part of the record that the SNR reads: the amplitude's coefficients and
+// fcut (values, in the same slots, without the phase's and every tangent,
+// whose arithmetic the compiler then drops) and the event's constants.  The
+// tau coefficients' tangents come from what the record held and are not read.
+template <int MODEL>
+GWF_HD void setup_event_snr(const gwf_waveform& w, const NetK& net, const double* par, int64_t ld, int64_t e,
+                            double* rec) {
+  const double Mc = par[0 * ld + e], eta = par[1 * ld + e];
+  const double chi1 = par[9 * ld + e], chi2 = par[10 * ld + e];
+  const D<1> Mcs = mkc<1>(Mc), etas = mkc<1>(eta), c1s = mkc<1>(chi1), c2s = mkc<1>(chi2);
+  if constexpr (MODEL == GWF_MODEL_IMRPHENOMD) {
+    pd_setup<1, PD_AMP, true>(Mcs, etas, c1s, c2s, 1.0, w.apply_fcut != 0, w.qnm_a, w.qnm_fring, w.qnm_fdamp, w.n_qnm, rec,
+                      SLOT, mkc<1>(1.0), mkc<1>(1.0));
+  } else if constexpr (MODEL == GWF_MODEL_IMRPHENOMD_NRTIDALV2) {
+    D<1> L1, L2;
+    lam12_from_lamt(mkc<1>(par[11 * ld + e]), mkc<1>(par[12 * ld + e]), etas, L1, L2);
+    const D<1> QM1 = quadmon(L1), QM2 = quadmon(L2);
+    pd_setup<1, PD_AMP, true>(Mcs, etas, c1s, c2s, 1.0, w.apply_fcut != 0, w.qnm_a, w.qnm_fring, w.qnm_fdamp, w.n_qnm, rec,
+                      SLOT, QM1, QM2);
+    nrt_setup<1, PD_AMP, true>(Mcs, etas, c1s, c2s, L1, L2, QM1, QM2, rec, SLOT);
+  } else {
+    rec[TF_MG * SLOT] = (Mcs * GMSUN_C3 / dpow(etas, 3. / 5.)).v;
+    rec[TF_AMP * SLOT] = tf2_amp_coeff(Mcs).v;
+    rec[TF_FCUT * SLOT] = tf2_fcut(w, Mc, eta, chi1, chi2);
+  }
+  setup_event_consts<MODEL>(net, par, ld, e, rec);
+}
+
 // Fills the event record: waveform coefficients (duals) + projection constants.
 template <int MODEL, int NT>
 GWF_HD void setup_event(const gwf_waveform& w, const NetK& net, const double* par, int64_t ld, int64_t e, double f0,
@@ -1395,9 +1423,13 @@ GWF_HD void pc_consume_semi(const NetK& net, const double* rec, int base, int re
 // walk: the amplitude, tau(f) and the PSD segments are evaluated once per
 // frequency and shared by the sites.  acc[a] accumulates physical arm a
 // (a < MAXA, the network's arm count rounded up to a compile-time bound).
-template <int MODEL, int MAXA = GWF_MAX_ARMS>
-GWF_HD void snr_event(const gwf_waveform& w, const NetK& net, const double* rec, int res, int lane, int nlanes,
-                      double acc[MAXA]) {
+// Walks the event's grid in chunks of nlanes points and runs put(k, wS, |h|^2)
+// for every arm k of the lane's point in the chunks c % parts == part, and
+// after(c) after every chunk.  (Every part walks the whole grid, so that its
+// points do not depend on the split.)
+template <int MODEL, int MAXA, class Put, class After>
+GWF_HD void snr_points(const gwf_waveform& w, const NetK& net, const double* rec, int res, int lane, int nlanes,
+                       int part, int parts, Put&& put, After&& after) {
   const double* ev = rec + REC_EV;
   const double a = log10(net.fmin);
   const double b = log10(fcut_eff(ev[EV_FCUT], net.fmax));
@@ -1405,53 +1437,66 @@ GWF_HD void snr_event(const gwf_waveform& w, const NetK& net, const double* rec,
   const bool earth = net.any_earth != 0;
   GridWalk<false> gw;
   gw.init(a, b, res, lane, nlanes);
+  int turn = 0;  // the chunk's number modulo parts
   for (int base = 0; base < res; base += nlanes) {
     const int i = base + lane;
     double f, wt, lnf;
     gw.step(base, res, &f, &wt, &lnf);
-    if (i >= res) continue;
-    PsdPre pre0, pre1;
-    psd_prefetch(net.psd[0], f, lnf, pre0);
-    if (net.n_psd > 1) psd_prefetch(net.psd[1], f, lnf, pre1);
-    double tau;
-    const double Av = wf_amp_tau_val<MODEL>(w, rec, f, lnf, earth, &tau) * idL;
-    double cdel, sdel;
-    earth_delta(earth, tau, &cdel, &sdel);
-    int cur_site = -1, cur_psd = -1;
-    double wS = 0.0, P1 = 0.0, P2 = 0.0;
-    Geo g;
+    const bool mine = turn == part;
+    turn = turn + 1 == parts ? 0 : turn + 1;
+    if (mine && i < res) {
+      PsdPre pre0, pre1;
+      psd_prefetch(net.psd[0], f, lnf, pre0);
+      if (net.n_psd > 1) psd_prefetch(net.psd[1], f, lnf, pre1);
+      double tau;
+      const double Av = wf_amp_tau_val<MODEL>(w, rec, f, lnf, earth, &tau) * idL;
+      double cdel, sdel;
+      earth_delta(earth, tau, &cdel, &sdel);
+      int cur_site = -1, cur_psd = -1;
+      double wS = 0.0, P1 = 0.0, P2 = 0.0;
+      Geo g;
 #pragma unroll
-    for (int k = 0; k < MAXA; ++k) {
-      if (k < net.n_arms) {
-        const ArmK& A = net.arm[k];
-        const int s = A.site;
-        if (s != cur_site) {
-          const SiteK& S = net.site[s];
-          const double* sc = rec + REC_SITE + s * SC_COUNT;
-          if (S.psd != cur_psd) {
-            double Sf;
-            if (S.psd == 0)
-              Sf = psd_finish(net.psd[0], f, lnf, pre0);
-            else if (S.psd == 1)
-              Sf = psd_finish(net.psd[1], f, lnf, pre1);
-            else
-              Sf = psd_at(net.psd[S.psd], f, lnf);
-            wS = wt / Sf;
-            cur_psd = S.psd;
+      for (int k = 0; k < MAXA; ++k) {
+        if (k < net.n_arms) {
+          const ArmK& A = net.arm[k];
+          const int s = A.site;
+          if (s != cur_site) {
+            const SiteK& S = net.site[s];
+            const double* sc = rec + REC_SITE + s * SC_COUNT;
+            if (S.psd != cur_psd) {
+              double Sf;
+              if (S.psd == 0)
+                Sf = psd_finish(net.psd[0], f, lnf, pre0);
+              else if (S.psd == 1)
+                Sf = psd_finish(net.psd[1], f, lnf, pre1);
+              else
+                Sf = psd_at(net.psd[S.psd], f, lnf);
+              wS = wt / Sf;
+              cur_psd = S.psd;
+            }
+            site_geo<false>(S, sc, ev, site_tn(S.motion, tc, tau), cdel, sdel, g);
+            P1 = sc[SC_P1];
+            P2 = sc[SC_P2];
+            cur_site = s;
           }
-          site_geo<false>(S, sc, ev, site_tn(S.motion, tc, tau), cdel, sdel, g);
-          P1 = sc[SC_P1];
-          P2 = sc[SC_P2];
-          cur_site = s;
+          const double aa = A.s2x * g.Sa - A.c2x * g.Ca;
+          const double bb = A.c2x * g.Cb + A.s2x * g.Sb;
+          const double Ap = Av * (aa * P1 + bb * P2) * cp;
+          const double Ac = Av * (bb * P1 - aa * P2) * cc;
+          put(k, wS, Ap * Ap + Ac * Ac);
         }
-        const double aa = A.s2x * g.Sa - A.c2x * g.Ca;
-        const double bb = A.c2x * g.Cb + A.s2x * g.Sb;
-        const double Ap = Av * (aa * P1 + bb * P2) * cp;
-        const double Ac = Av * (bb * P1 - aa * P2) * cc;
-        acc[k] += wS * (Ap * Ap + Ac * Ac);
       }
     }
+    after(base / nlanes);
   }
+}
+
+template <int MODEL, int MAXA = GWF_MAX_ARMS>
+GWF_HD void snr_event(const gwf_waveform& w, const NetK& net, const double* rec, int res, int lane, int nlanes,
+                      double acc[MAXA]) {
+  snr_points<MODEL, MAXA>(
+      w, net, rec, res, lane, nlanes, 0, 1, [&](int k, double wS, double h2) { acc[k] = fma(wS, h2, acc[k]); },
+      [](int) {});
 }
 
 // ------------------------------------------------------------- strain body

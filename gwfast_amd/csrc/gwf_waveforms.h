@@ -259,7 +259,11 @@ GWF_HD X pd_phi_piecewise(const PdPhase<T>& c, const X& x, bool apply_fcut) {
 // Per-event IMRPhenomD setup. Mc, eta, chi1, chi2 are seeded duals (or
 // doubles); f0 is the frequency whose M*G*f0 is fRef (grid minimum or the
 // model's fixed fRef); rec receives PD_COUNT entries of stride (N+1).
-template <int N>
+// PARTS: the slots written, PD_AMP (the amplitude's, M G and fcut) and
+// PD_PHASE (the rest); the compiler drops the arithmetic of what is not
+// written.  VALUES: without tangents.
+constexpr int PD_AMP = 1, PD_PHASE = 2;
+template <int N, int PARTS = PD_AMP | PD_PHASE, bool VALUES = false>
 GWF_HD void pd_setup(const D<N>& Mc, const D<N>& eta, const D<N>& chi1, const D<N>& chi2, double f0,
                      bool apply_fcut, const double* qa, const double* qfr, const double* qfd, int nq,
                      double* rec, int stride, const D<N>& QM1, const D<N>& QM2, int tk = -1) {
@@ -385,17 +389,26 @@ GWF_HD void pd_setup(const D<N>& Mc, const D<N>& eta, const D<N>& chi1, const D<
   // starts: none of them is live past this point but fring and fdamp, which
   // shortens the live ranges through the collocation solve below.
   double* r = rec;
-  auto put = [&](int slot, const T& x) { std_tk(r + slot * stride, x, tk); };
+  auto putp = [&](int slot, const T& x) {
+    if constexpr ((PARTS & PD_PHASE) != 0) std_tk(r + slot * stride, x, tk);
+  };
+  auto put = [&](int slot, const T& x) {
+    if constexpr (VALUES)
+      r[slot * stride] = x.v;
+    else if constexpr ((PARTS & PD_AMP) != 0)
+      std_tk(r + slot * stride, x, tk);
+  };
   put(PD_MG, MG);
-  put(PD_ETA, eta);
-  put(PD_PIP, c.pip); put(PD_P23, c.p23); put(PD_P13, c.p13); put(PD_P13L, c.p13l); put(PD_PLOG, c.plog);
-  put(PD_PM13, c.pm13); put(PD_PM23, c.pm23); put(PD_PM1, c.pm1); put(PD_PM53, c.pm53);
-  put(PD_S1, c.s1); put(PD_S43, c.s43); put(PD_S53, c.s53); put(PD_S2, c.s2);
-  put(PD_B1, beta1); put(PD_B2, beta2); put(PD_B3, beta3); put(PD_C1I, C1Int); put(PD_C2I, C2Int);
-  put(PD_A1, alpha1); put(PD_A2, alpha2); put(PD_A3, alpha3); put(PD_A4, alpha4); put(PD_A5, alpha5);
-  put(PD_C1M, C1MRD); put(PD_C2M, C2MRD);
-  put(PD_FRING, fring); put(PD_FDAMP, fdamp); put(PD_FMRDJ, fMRDJoin); put(PD_T0, t0); put(PD_FREF, fRef);
-  put(PD_PHIREF, phiRef);
+  put(PD_FRING, fring); put(PD_FDAMP, fdamp);
+  putp(PD_ETA, eta);
+  putp(PD_PIP, c.pip); putp(PD_P23, c.p23); putp(PD_P13, c.p13); putp(PD_P13L, c.p13l); putp(PD_PLOG, c.plog);
+  putp(PD_PM13, c.pm13); putp(PD_PM23, c.pm23); putp(PD_PM1, c.pm1); putp(PD_PM53, c.pm53);
+  putp(PD_S1, c.s1); putp(PD_S43, c.s43); putp(PD_S53, c.s53); putp(PD_S2, c.s2);
+  putp(PD_B1, beta1); putp(PD_B2, beta2); putp(PD_B3, beta3); putp(PD_C1I, C1Int); putp(PD_C2I, C2Int);
+  putp(PD_A1, alpha1); putp(PD_A2, alpha2); putp(PD_A3, alpha3); putp(PD_A4, alpha4); putp(PD_A5, alpha5);
+  putp(PD_C1M, C1MRD); putp(PD_C2M, C2MRD);
+  putp(PD_FMRDJ, fMRDJoin); putp(PD_T0, t0); putp(PD_FREF, fRef);
+  putp(PD_PHIREF, phiRef);
 
   // Amplitude (waveforms.py:1188-1248); fpeak with fabs on the first branch only (1193)
   const T fpeakA = (val(gamma2) >= 1.0) ? dfabs(fring - (fdamp * gamma3) / gamma2)
@@ -540,7 +553,7 @@ GWF_HD void pd_setup(const D<N>& Mc, const D<N>& eta, const D<N>& chi1, const D<
 
   // fcut = 0.2 / (Mc G / eta^(3/5)) (waveforms.py:1333)
   put(PD_FCUT, mkc<N>(0.2 / (Mc.v * GMSUN_C3 / pow(eta.v, 3. / 5.))));
-  put(PD_IETA, 1.0 / eta);
+  putp(PD_IETA, 1.0 / eta);
 }
 
 template <int N>
@@ -848,6 +861,12 @@ GWF_HD double tf2_fcut(const gwf_waveform& w, double Mc, double eta, double chi1
 // (Mc, eta, chi1z, chi2z, ecc); the tidal one has N = 6.
 constexpr bool tf2_eccentric(int N) { return N == 5 || N == 7; }  // 7: tidal and eccentric
 
+// sqrt(5/24) pi^(-2/3) clightGpc (G Mc)^(5/6)  (waveforms.py:875, without 1/dL)
+template <class T>
+GWF_HD T tf2_amp_coeff(const T& Mc) {
+  return sqrt(5. / 24.) * pow(PI, -2. / 3.) * CLIGHT_GPC * dpow(GMSUN_C3 * Mc, 5. / 6.);
+}
+
 template <int N>
 GWF_HD void tf2_setup(const gwf_waveform& w, const D<N>& Mc, const D<N>& eta, const D<N>& chi1, const D<N>& chi2,
                       const D<N>& Lamt, const D<N>& delLam, double* rec, int stride, const D<N>& ecc = D<N>(),
@@ -902,8 +921,7 @@ GWF_HD void tf2_setup(const gwf_waveform& w, const D<N>& Mc, const D<N>& eta, co
   put(TF_C10, TF2OA * t10);
   put(TF_C12, TF2OA * t12);
   put(TF_PHIR, mkc<N>(phiR - PI * 0.25));
-  // sqrt(5/24) pi^(-2/3) clightGpc (G Mc)^(5/6)  (waveforms.py:875, without 1/dL)
-  put(TF_AMP, sqrt(5. / 24.) * pow(PI, -2. / 3.) * CLIGHT_GPC * dpow(GMSUN_C3 * Mc, 5. / 6.));
+  put(TF_AMP, tf2_amp_coeff(Mc));
   put(TF_FCUT, mkc<N>(tf2_fcut(w, Mc.v, eta.v, chi1.v, chi2.v)));
   if (tf2_eccentric(N)) {
     // low-eccentricity 3PN phase of arXiv:1605.00304 as written in waveforms.py:814-845;
@@ -1014,7 +1032,7 @@ GWF_HD double nrt_fcut(double Mc, double eta, double Lt, double dLm) {
 // The NRTidalv2 slots of an event record (after pd_setup with the same
 // quadrupole moments): tidal-phase factor, 3.5PN SS + SSS coefficient,
 // tidal-amplitude factor, merger frequency, and the model's fcut.
-template <int N>
+template <int N, int PARTS = PD_AMP | PD_PHASE, bool VALUES = false>
 GWF_HD void nrt_setup(const D<N>& Mc, const D<N>& eta, const D<N>& chi1, const D<N>& chi2, const D<N>& L1,
                       const D<N>& L2, const D<N>& QM1, const D<N>& QM2, double* rec, int stride, int tk = -1) {
   typedef D<N> T;
@@ -1040,9 +1058,16 @@ GWF_HD void nrt_setup(const D<N>& Mc, const D<N>& eta, const D<N>& chi1, const D
   // Overallamp without 1/dL (waveforms.py:1248) times 2 sqrt(pi/5) and -9 kappa2T
   const T OA = 2. * sqrt(5. / (64. * PI)) * M * GMSUN_C2_GPC * M * GMSUN_C3;
   const T fm = nrt_fmerger(eta, Seta, kappa2T);
-  auto put = [&](int slot, const T& x) { std_tk(rec + slot * stride, x, tk); };
-  put(PD_TPH, -kappa2T * 2.4375 / (m1ByM * m2ByM));
-  put(PD_SSS, (SS + SSS) * TF2OA);
+  auto put = [&](int slot, const T& x) {
+    if constexpr (VALUES)
+      rec[slot * stride] = x.v;
+    else if constexpr ((PARTS & PD_AMP) != 0)
+      std_tk(rec + slot * stride, x, tk);
+  };
+  if constexpr ((PARTS & PD_PHASE) != 0) {
+    std_tk(rec + PD_TPH * stride, -kappa2T * 2.4375 / (m1ByM * m2ByM), tk);
+    std_tk(rec + PD_SSS * stride, (SS + SSS) * TF2OA, tk);
+  }
   put(PD_TAMP, OA * (2. * sqrt(PI / 5.)) * (-9.0 * kappa2T));
   put(PD_FMERG, fm);
   put(PD_FCUT, mkc<N>((1.2 * fm.v) / (M.v * GMSUN_C3)));

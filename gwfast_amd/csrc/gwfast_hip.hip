@@ -211,6 +211,17 @@ __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const d
   }
 }
 
+// The SNR's records (setup_event_snr), one lane per event: values of the
+// amplitude's slots alone, where k_setup's tangents and phase bound a large
+// batch (10^5 IMRPhenomD events: k_setup 310 us, this 81) and its chain a
+// small one (100 tidal TaylorF2 events 12 us, 7).
+template <int MODEL>
+__global__ __launch_bounds__(256) void k_setup_snr(gwf_waveform w, NetK net, const double* __restrict__ par, int64_t ld,
+                                                   int64_t n_ev, double* __restrict__ rec) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < n_ev) setup_event_snr<MODEL>(w, net, par, ld, e, rec + e * (int64_t)REC_DOUBLES);
+}
+
 #ifndef GWF_FISHER_MIN_BLOCKS
 #define GWF_FISHER_MIN_BLOCKS 1
 #endif
@@ -1231,7 +1242,15 @@ __global__ void k_zero_u32(unsigned int* p, int n) {
   if (i < n) p[i] = 0u;
 }
 
-// 3 waves per SIMD (<= 168 VGPRs): measured fastest for the 5-arm network
+// The values, constants and sites of an event's record that the SNR reads,
+// into LDS (the values alone of the waveform's slots).
+__device__ __forceinline__ void snr_record(const double* __restrict__ rg, double* rl, int n_sites, int t, int nt) {
+  for (int q = t; q < REC_EV / SLOT; q += nt) rl[q * SLOT] = rg[q * SLOT];
+  for (int q = REC_EV + t; q < REC_SITE + n_sites * SC_COUNT; q += nt) rl[q] = rg[q];
+}
+
+// One wave per event, 3 waves per SIMD (<= 168 VGPRs): measured fastest for
+// the 5-arm network
 template <int MODEL, int MAXA>
 __global__ __launch_bounds__(256, 3) void k_snr(gwf_waveform w, NetK net, const double* __restrict__ rec, int64_t n_ev,
                                              const int* __restrict__ res_ev, double* __restrict__ out) {
@@ -1243,8 +1262,7 @@ __global__ __launch_bounds__(256, 3) void k_snr(gwf_waveform w, NetK net, const 
   // 37.5 ms at 10^6 events x 2000 f)
   __shared__ double recs[WAVES_PER_BLOCK][REC_DOUBLES];
   double* rl = recs[threadIdx.x >> 6];
-  const double* rg = rec + e * (int64_t)REC_DOUBLES;
-  for (int q = lane; q < REC_DOUBLES; q += 64) rl[q] = rg[q];
+  snr_record(rec + e * (int64_t)REC_DOUBLES, rl, net.n_sites, lane, 64);
   const double* r = rl;
   double acc[MAXA];
 #pragma unroll
@@ -1256,6 +1274,47 @@ __global__ __launch_bounds__(256, 3) void k_snr(gwf_waveform w, NetK net, const 
       const double v = wave_sum(acc[k]);
       if (lane == 0) out[(int64_t)k * n_ev + e] = v;
     }
+  }
+}
+
+// A block of SNR_WAVES waves per event, for batches that would leave SIMDs
+// without a wave: wave q takes chunk q of every SNR_WAVES, its points' weights
+// and |h|^2 go to LDS, and wave k adds arm k's in chunk order, as k_snr does
+// (the same sums in the same order).  Up to MAXA = 8 arms: the LDS holds 64 KB
+// of them.  100 tidal TaylorF2 events x 1000 points, three arms: 34 us with a
+// wave per event (16 chunks one after another), 18 us with a block.
+constexpr int SNR_WAVES = 8;
+template <int MODEL>
+__global__ __launch_bounds__(64 * SNR_WAVES, 3) void k_snr_split(gwf_waveform w, NetK net,
+                                                                 const double* __restrict__ rec, int64_t n_ev,
+                                                                 const int* __restrict__ res_ev,
+                                                                 double* __restrict__ out) {
+  constexpr int MAXA = SNR_WAVES;
+  __shared__ double rl[REC_DOUBLES];
+  __shared__ double2 term[SNR_WAVES][MAXA][64];
+  const int64_t e = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  snr_record(rec + e * (int64_t)REC_DOUBLES, rl, net.n_sites, threadIdx.x, blockDim.x);
+  __syncthreads();
+  const int res = res_ev ? min(max(__builtin_amdgcn_readfirstlane(res_ev[e]), 2), 1 << 30) : net.res;
+  double acc = 0.0;
+  const int last = (res - 1) / 64;
+  snr_points<MODEL, MAXA>(
+      w, net, rl, res, lane, 64, wave, SNR_WAVES,
+      [&](int k, double wS, double h2) { term[wave][k][lane] = make_double2(wS, h2); },
+      [&](int c) {
+        if (c % SNR_WAVES != SNR_WAVES - 1 && c != last) return;
+        __syncthreads();
+        if (wave < net.n_arms) {
+          const int c0 = c - c % SNR_WAVES;
+          for (int q = c0; q <= c; ++q)
+            if (64 * q + lane < res) acc = fma(term[q - c0][wave][lane].x, term[q - c0][wave][lane].y, acc);
+        }
+        __syncthreads();
+      });
+  if (wave < net.n_arms) {
+    const double v = wave_sum(acc);
+    if (lane == 0) out[(int64_t)wave * n_ev + e] = v;
   }
 }
 
@@ -2626,6 +2685,13 @@ void launch_fisher_ragged(const gwf_waveform* wf, dim3 grid, dim3 block, hipStre
                        res_ev, arm, counter, out);
 }
 
+int cu_count(int* n_cu) {
+  int dev = 0;
+  const int rc = hip_check(hipGetDevice(&dev), "hipGetDevice");
+  if (rc) return rc;
+  return hip_check(hipDeviceGetAttribute(n_cu, hipDeviceAttributeMultiprocessorCount, dev), "CU count");
+}
+
 // The network Fisher on producer / consumer pairs (k_fisher_pq): one
 // resident block per CU, then the NaN fill that reports an expired wait.
 // counter: two words, zeroed here.
@@ -2633,10 +2699,8 @@ template <bool LIN, bool RAGGED, int MODE = PQ_SUM>
 int launch_fisher_pq(const gwf_waveform* wf, hipStream_t st, const NetK& net_in, const double* rec, int64_t n_ev,
                      const int32_t* res_ev, unsigned int* counter, double* out, int P,
                      const uint32_t* arm_mask = nullptr) {
-  int dev = 0, n_cu = 0;
-  int rc = hip_check(hipGetDevice(&dev), "hipGetDevice");
-  if (rc) return rc;
-  rc = hip_check(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev), "CU count");
+  int n_cu = 0;
+  int rc = cu_count(&n_cu);
   if (rc) return rc;
   hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, counter, 2);
   const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((n_ev + PC_EPB - 1) / PC_EPB, n_cu));
@@ -2702,6 +2766,24 @@ int launch_setup(const gwf_waveform* wf, const NetK& net, const double* par, int
   else
     hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 4>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
                        rec);
+  return hip_check(hipGetLastError(), "setup launch");
+}
+
+// The records of an SNR call on its own (launch_setup's where a caller
+// prepares them: they may go to the Fisher kernels).  One lane per event;
+// blocks as launch_setup's.
+int launch_setup_snr(const gwf_waveform* wf, const NetK& net, const double* par, int64_t ld, int64_t n_ev,
+                     double* rec, hipStream_t st) {
+  const int bs = n_ev <= 65536 * 4 ? 64 : 256;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n_ev + bs - 1) / bs)), dim3(bs), 0, st, *wf, net, par, ld, n_ev, rec);
+  };
+  if (wf->model == GWF_MODEL_IMRPHENOMD)
+    go(k_setup_snr<GWF_MODEL_IMRPHENOMD>);
+  else if (wf->model == GWF_MODEL_IMRPHENOMD_NRTIDALV2)
+    go(k_setup_snr<GWF_MODEL_IMRPHENOMD_NRTIDALV2>);
+  else
+    go(k_setup_snr<GWF_MODEL_TAYLORF2>);
   return hip_check(hipGetLastError(), "setup launch");
 }
 
@@ -2867,8 +2949,9 @@ int gwf_waveform_eval(const gwf_waveform* wf, const double* params, int64_t ld, 
   return hip_check(hipGetLastError(), "gwf_waveform_eval launch");
 }
 
-int gwf_prepare(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, const double* params, int64_t ld,
-                int64_t n_ev, int32_t res, void* workspace, size_t ws_bytes, void* stream) {
+static int prepare_impl(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, const double* params,
+                        int64_t ld, int64_t n_ev, int32_t res, bool snr, void* workspace, size_t ws_bytes,
+                        void* stream) {
   int rc = check_common(wf, params, ld, n_ev, workspace, ws_bytes);
   if (rc) return rc;
   if (res < 2) return fail(-EINVAL, "res must be >= 2");
@@ -2876,7 +2959,13 @@ int gwf_prepare(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det,
   rc = build_net_checked(dets, n_det, res, net);
   if (rc) return rc;
   if (n_ev == 0) return 0;
+  if (snr) return launch_setup_snr(wf, net, params, ld, n_ev, (double*)workspace, (hipStream_t)stream);
   return launch_setup(wf, net, params, ld, n_ev, nullptr, 0, (double*)workspace, (hipStream_t)stream);
+}
+
+int gwf_prepare(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, const double* params, int64_t ld,
+                int64_t n_ev, int32_t res, void* workspace, size_t ws_bytes, void* stream) {
+  return prepare_impl(wf, dets, n_det, params, ld, n_ev, res, false, workspace, ws_bytes, stream);
 }
 
 static int snr_prepared_impl(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, int64_t n_ev, int32_t res,
@@ -2893,18 +2982,31 @@ static int snr_prepared_impl(const gwf_waveform* wf, const gwf_detector* dets, i
   if (n_ev == 0) return 0;
   if (!snrsq_out) return fail(-EINVAL, "snrsq_out is NULL");
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)((n_ev + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK)), block(BLOCK);
+  // no more events than CUs: a block of eight waves for each
+  const bool small = net.n_arms <= 8;  // per-arm accumulators held in registers
+  int n_cu = 0;
+  rc = cu_count(&n_cu);
+  if (rc) return rc;
+  const bool split = small && n_ev <= n_cu;
+  const dim3 grid((unsigned)(split ? n_ev : (n_ev + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK));
+  const dim3 block(split ? 64 * SNR_WAVES : BLOCK);
   const double* rec = (const double*)workspace;
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, block, 0, st, *wf, net, rec, n_ev, res_ev, snrsq_out);
   };
-  const bool small = net.n_arms <= 8;  // per-arm accumulators held in registers
+  auto pick = [&](auto model) {
+    constexpr int MODEL = decltype(model)::value;
+    if (split)
+      go(k_snr_split<MODEL>);
+    else
+      small ? go(k_snr<MODEL, 8>) : go(k_snr<MODEL, GWF_MAX_ARMS>);
+  };
   if (wf->model == GWF_MODEL_IMRPHENOMD)
-    small ? go(k_snr<GWF_MODEL_IMRPHENOMD, 8>) : go(k_snr<GWF_MODEL_IMRPHENOMD, GWF_MAX_ARMS>);
+    pick(std::integral_constant<int, GWF_MODEL_IMRPHENOMD>{});
   else if (wf->model == GWF_MODEL_IMRPHENOMD_NRTIDALV2)
-    small ? go(k_snr<GWF_MODEL_IMRPHENOMD_NRTIDALV2, 8>) : go(k_snr<GWF_MODEL_IMRPHENOMD_NRTIDALV2, GWF_MAX_ARMS>);
+    pick(std::integral_constant<int, GWF_MODEL_IMRPHENOMD_NRTIDALV2>{});
   else
-    small ? go(k_snr<GWF_MODEL_TAYLORF2, 8>) : go(k_snr<GWF_MODEL_TAYLORF2, GWF_MAX_ARMS>);
+    pick(std::integral_constant<int, GWF_MODEL_TAYLORF2>{});
   return hip_check(hipGetLastError(), "gwf_snr launch");
 }
 
@@ -3009,7 +3111,7 @@ int gwf_fisher_arms(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_
 
 int gwf_snr(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, const double* params, int64_t ld,
             int64_t n_ev, int32_t res, double* snrsq_out, void* workspace, size_t ws_bytes, void* stream) {
-  int rc = gwf_prepare(wf, dets, n_det, params, ld, n_ev, res, workspace, ws_bytes, stream);
+  int rc = prepare_impl(wf, dets, n_det, params, ld, n_ev, res, true, workspace, ws_bytes, stream);
   if (rc) return rc;
   return gwf_snr_prepared(wf, dets, n_det, n_ev, res, snrsq_out, workspace, ws_bytes, stream);
 }
@@ -3037,7 +3139,7 @@ int gwf_snr_ragged(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_d
                    int64_t n_ev, const int32_t* res_ev, double* snrsq_out, void* workspace, size_t ws_bytes,
                    void* stream) {
   if (n_ev > 0 && !res_ev) return fail(-EINVAL, "res_ev is NULL");
-  int rc = gwf_prepare(wf, dets, n_det, params, ld, n_ev, 2, workspace, ws_bytes, stream);
+  int rc = prepare_impl(wf, dets, n_det, params, ld, n_ev, 2, true, workspace, ws_bytes, stream);
   if (rc) return rc;
   return snr_prepared_impl(wf, dets, n_det, n_ev, 2, res_ev, snrsq_out, workspace, ws_bytes, stream);
 }

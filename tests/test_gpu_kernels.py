@@ -201,3 +201,42 @@ def test_strain_split_over_an_events_points(P, n, nf):
     hm, Jm = S.strain_device(sig, rows.repeat(1, k).contiguous(), f.repeat(1, k).contiguous(), 0)
     assert np.array_equal(h.cpu().numpy(), hm[:, :n].cpu().numpy())
     assert np.array_equal(J.cpu().numpy(), Jm[:, :n].cpu().numpy())
+
+
+SITES_10_ARMS = ['ETS', 'ETMR', 'CE1Id', 'CE2NM', 'Virgo', 'KAGRA']
+
+
+@pytest.mark.parametrize('P', [11, 12, 13, 'NRTidalv2'])
+@pytest.mark.parametrize('arms', [5, 10])
+@pytest.mark.parametrize('res', [2, 64, 65, 513, 1000])
+def test_snr_of_few_and_many_events(P, arms, res):
+    """Few events (a block of eight waves each, up to 8 arms) against the same
+    events among 1000 (a wave each), and the SNR's own records against those a
+    caller prepares for the Fisher kernels: the same terms in the same order up
+    to the compiler's contractions, a few ulp of each, so 10^3 2^-52 relative."""
+    import torch
+    from tests._common import NET_C1, hip_net
+    from gwfast_amd import _engine as E, _native as N, gwfastGlobals as glob, signal as S
+    from gwfast_amd.waveforms import IMRPhenomD_NRTidalv2
+    wf = IMRPhenomD_NRTidalv2() if P == 'NRTidalv2' else _wf(P)
+    tidal = P in (13, 'NRTidalv2')
+    n = 5
+    rows = E.to_dev(E.param_rows(_events(13 if tidal else P, n, 8), tidal, P == 12))
+    net = NET_C1 if arms == 5 else [(s, glob.PSD_ET if s[0] == 'E' else glob.PSD_CE) for s in SITES_10_ARMS]
+    sigs = list(hip_net(wf, net, True).signals.values())
+    few_len = np.array([res, 2, 64, max(2, res // 2), res], dtype=np.int32)
+
+    def close(a, b):
+        return bool(((a - b).abs() <= 1e3 * 2. ** -52 * b).all())
+
+    for ln, tile in ((res, False), (few_len, True)):
+        few = S.snr_sq_device(sigs, rows, ln)
+        many = S.snr_sq_device(sigs, rows.repeat(1, 200).contiguous(), np.tile(ln, 200) if tile else ln)
+        assert few.shape == (arms, n) and close(few, many[:, :n])
+    ws, nb = E.workspace(n)
+    dets = S._dets(sigs)
+    E.call('gwf_prepare', wf.c_struct(), dets, len(sigs), N.ptr(rows), rows.stride(0), n, res, N.ptr(ws), nb,
+           N.stream_ptr())
+    out = torch.empty((arms, n), dtype=torch.float64, device='cuda')
+    E.call('gwf_snr_prepared', wf.c_struct(), dets, len(sigs), n, res, N.ptr(out), N.ptr(ws), nb, N.stream_ptr())
+    assert close(S.snr_sq_device(sigs, rows, res), out)
