@@ -278,7 +278,8 @@ GWF_HD constexpr bool is_pd(int model) {
 // The same arithmetic as the NT-tangent evaluation, in a fifth of the
 // registers, so the dependent chain of the collocation solve no longer
 // spills.
-template <int MODEL>
+// PARTS: the slots written (pd_setup).
+template <int MODEL, int PARTS>
 GWF_HD void setup_waveform_split(const gwf_waveform& w, const double* par, int64_t ld, int64_t e, double f0,
                                  double* rec, int tk) {
   static_assert(is_pd(MODEL), "split setup: IMRPhenomD models");
@@ -288,20 +289,21 @@ GWF_HD void setup_waveform_split(const gwf_waveform& w, const double* par, int64
   const double f0u = (w.fref > 0.0) ? w.fref : f0;
   const D<1> Mcs = seed(Mc, 0), etas = seed(eta, 1), c1s = seed(chi1, 2), c2s = seed(chi2, 3);
   if (MODEL == GWF_MODEL_IMRPHENOMD) {
-    pd_setup<1>(Mcs, etas, c1s, c2s, f0u, w.apply_fcut != 0, w.qnm_a, w.qnm_fring, w.qnm_fdamp, w.n_qnm, rec, SLOT,
+    pd_setup<1, PARTS>(Mcs, etas, c1s, c2s, f0u, w.apply_fcut != 0, w.qnm_a, w.qnm_fring, w.qnm_fdamp, w.n_qnm, rec, SLOT,
                 mkc<1>(1.0), mkc<1>(1.0), tk);
   } else {
     D<1> L1, L2;
     lam12_from_lamt(seed(par[11 * ld + e], 4), seed(par[12 * ld + e], 5), etas, L1, L2);
     const D<1> QM1 = quadmon(L1), QM2 = quadmon(L2);
-    pd_setup<1>(Mcs, etas, c1s, c2s, f0u, w.apply_fcut != 0, w.qnm_a, w.qnm_fring, w.qnm_fdamp, w.n_qnm, rec, SLOT,
+    pd_setup<1, PARTS>(Mcs, etas, c1s, c2s, f0u, w.apply_fcut != 0, w.qnm_a, w.qnm_fring, w.qnm_fdamp, w.n_qnm, rec, SLOT,
                 QM1, QM2, tk);
-    nrt_setup<1>(Mcs, etas, c1s, c2s, L1, L2, QM1, QM2, rec, SLOT, tk);
+    nrt_setup<1, PARTS>(Mcs, etas, c1s, c2s, L1, L2, QM1, QM2, rec, SLOT, tk);
   }
 }
 
-template <int MODEL>
-GWF_HD void setup_event_consts(const NetK& net, const double* par, int64_t ld, int64_t e, double* rec);
+// mg: M G and its tangents d/dMc, d/deta; fcut: the model's
+GWF_HD void setup_event_consts(const NetK& net, const double* par, int64_t ld, int64_t e, const double* mg, double fcut,
+                               double* rec);
 
 // The part of the record that the SNR reads: the amplitude's coefficients and
 // fcut (values, in the same slots, without the phase's and every tangent,
@@ -328,7 +330,8 @@ GWF_HD void setup_event_snr(const gwf_waveform& w, const NetK& net, const double
     rec[TF_AMP * SLOT] = tf2_amp_coeff(Mcs).v;
     rec[TF_FCUT * SLOT] = tf2_fcut(w, Mc, eta, chi1, chi2);
   }
-  setup_event_consts<MODEL>(net, par, ld, e, rec);
+  constexpr int MGS = is_pd(MODEL) ? (int)PD_MG : (int)TF_MG, FCS = is_pd(MODEL) ? (int)PD_FCUT : (int)TF_FCUT;
+  setup_event_consts(net, par, ld, e, rec + MGS * SLOT, rec[FCS * SLOT], rec);
 }
 
 // Fills the event record: waveform coefficients (duals) + projection constants.
@@ -365,7 +368,20 @@ GWF_HD void setup_event(const gwf_waveform& w, const NetK& net, const double* pa
     tf2_setup<NT>(w, mkseed<NT>(Mc, 0), mkseed<NT>(eta, 1), mkseed<NT>(chi1, 2), mkseed<NT>(chi2, 3),
                   mkseed<NT>(Lt, 4), mkseed<NT>(dLm, 5), rec, SLOT);
   }
-  setup_event_consts<MODEL>(net, par, ld, e, rec);
+  constexpr int MGS = is_pd(MODEL) ? (int)PD_MG : (int)TF_MG, FCS = is_pd(MODEL) ? (int)PD_FCUT : (int)TF_FCUT;
+  setup_event_consts(net, par, ld, e, rec + MGS * SLOT, rec[FCS * SLOT], rec);
+}
+
+// setup_event_consts of an IMRPhenomD model, with M G and fcut of its own
+// instead of the waveform part's (pd_setup, nrt_setup).
+template <int MODEL>
+GWF_HD void setup_pd_consts(const NetK& net, const double* par, int64_t ld, int64_t e, double* rec) {
+  const double Mc = par[0 * ld + e], eta = par[1 * ld + e];
+  const D<2> MG = mkseed<2>(Mc, 0) / dpow(mkseed<2>(eta, 1), 3. / 5.) * GMSUN_C3;
+  const double mg[3] = {MG.v, MG.d[0], MG.d[1]};
+  const double fcut = MODEL == GWF_MODEL_IMRPHENOMD ? 0.2 / (Mc * GMSUN_C3 / pow(eta, 3. / 5.))
+                                                    : nrt_fcut(Mc, eta, par[11 * ld + e], par[12 * ld + e]);
+  setup_event_consts(net, par, ld, e, mg, fcut, rec);
 }
 
 // tau_star (waveforms.py:878-901, 1299-1322) as K v^-8 P(v), P the polynomial of the
@@ -447,8 +463,8 @@ GWF_HD double tau_star_ev_val(const double* ev, double v, double lv) {
 // The event constants of the record (after its waveform coefficients, whose
 // fcut it reads): inclination factors, 1/dL, tcoal, sky angles, ln(M G) and
 // its (Mc, eta) tangents, and the projection constants of every site.
-template <int MODEL>
-GWF_HD void setup_event_consts(const NetK& net, const double* par, int64_t ld, int64_t e, double* rec) {
+GWF_HD void setup_event_consts(const NetK& net, const double* par, int64_t ld, int64_t e, const double* mg, double fcut,
+                               double* rec) {
   const double Mc = par[0 * ld + e], eta = par[1 * ld + e], dL = par[2 * ld + e];
   const double theta = par[3 * ld + e], phi = par[4 * ld + e], iota = par[5 * ld + e];
   const double psi = par[6 * ld + e], tc = par[7 * ld + e];
@@ -465,10 +481,9 @@ GWF_HD void setup_event_consts(const NetK& net, const double* par, int64_t ld, i
   ev[EV_RA] = phi;
   ev[EV_CRA] = cos(phi);
   ev[EV_SRA] = sin(phi);
-  ev[EV_FCUT] = rec[(is_pd(MODEL) ? (int)PD_FCUT : (int)TF_FCUT) * SLOT];
+  ev[EV_FCUT] = fcut;
   {  // ln(M G f) = ln(M G) + ln f on the grids, whose ln f comes with f;
      // ln(M G) = ln Mc - (3/5) ln eta + ln G: tangents 1/Mc and -(3/5)/eta
-    const double* mg = rec + (is_pd(MODEL) ? (int)PD_MG : (int)TF_MG) * SLOT;
     ev[EV_LMG] = log(mg[0]);
     ev[EV_LMG_D0] = 1.0 / Mc;
     ev[EV_LMG_D1] = -0.6 / eta;

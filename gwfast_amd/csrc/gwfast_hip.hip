@@ -190,7 +190,13 @@ template <int MODEL, int NT>
 __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const double* __restrict__ par, int64_t ld,
                                                int64_t n_ev, bool own_grid, double* __restrict__ rec) {
   // IMRPhenomD models: NT lanes per event, lane tk evaluating tangent tk
-  // (setup_waveform_split); TaylorF2: one lane per event
+  // (setup_waveform_split), and grid row y the phase's coefficients, the
+  // amplitude's or the event's constants: three chains of about the same
+  // length, which as one bound every batch that does not fill the chip
+  // (IMRPhenomD, one chain and three: 1 to 1000 events 31 and 19 us, 10^4 42
+  // and 37, 3 x 10^4 87 and 93, 10^5 330 and 315; the same split at every
+  // size, so that a record does not depend on the batch).  TaylorF2: one lane
+  // per event
   constexpr int LPE = is_pd(MODEL) ? NT : 1;
   const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t e = tid / LPE;
@@ -204,8 +210,12 @@ __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const d
   }
   double* r = rec + e * (int64_t)REC_DOUBLES;
   if constexpr (is_pd(MODEL)) {
-    setup_waveform_split<MODEL>(w, par, ld, e, f0, r, tk);
-    if (tk == 0) setup_event_consts<MODEL>(net, par, ld, e, r);  // reads only lane 0's stores
+    if (blockIdx.y == 0)
+      setup_waveform_split<MODEL, PD_PHASE>(w, par, ld, e, f0, r, tk);
+    else if (blockIdx.y == 1)
+      setup_waveform_split<MODEL, PD_AMP>(w, par, ld, e, f0, r, tk);
+    else if (tk == 0)
+      setup_pd_consts<MODEL>(net, par, ld, e, r);
   } else {
     setup_event<MODEL, NT>(w, net, par, ld, e, f0, r);
   }
@@ -2741,7 +2751,7 @@ int launch_setup(const gwf_waveform* wf, const NetK& net, const double* par, int
   const int lpe = wf->model == GWF_MODEL_IMRPHENOMD ? 4 : (wf->model == GWF_MODEL_IMRPHENOMD_NRTIDALV2 ? 6 : 1);
   const int64_t nt = n_ev * lpe;
   const int bs = nt <= 65536 * 4 ? 64 : 256;
-  const dim3 grid((unsigned)((nt + bs - 1) / bs)), block(bs);
+  const dim3 grid((unsigned)((nt + bs - 1) / bs), is_pd(wf->model) ? 3u : 1u), block(bs);
   // the grid minimum is the reference frequency of the models that have none set
   const bool own_grid = fgrid && (is_pd(wf->model) ? !(wf->fref > 0.0) : (wf->is_eccentric && !(wf->fref_ecc > 0.0)));
   if (own_grid) {
