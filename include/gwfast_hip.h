@@ -89,7 +89,9 @@ int gwf_abi_version(void);
 const char* gwf_last_error(void);
 
 /* Bytes of device workspace the calls below need for n_ev events
- * (per-event coefficient records, then 256 bytes of queue counters). */
+ * (per-event coefficient records, 256 bytes of queue counters, and 4 bytes
+ * per event for the order of a ragged batch; the records and counters alone
+ * are taken too, the events of a ragged batch then being run as they come). */
 size_t gwf_workspace_bytes(int64_t n_ev);
 
 /* Number of interferometer arms of a network: L -> 1, T -> 3. */

@@ -240,3 +240,26 @@ def test_snr_of_few_and_many_events(P, arms, res):
     out = torch.empty((arms, n), dtype=torch.float64, device='cuda')
     E.call('gwf_snr_prepared', wf.c_struct(), dets, len(sigs), n, res, N.ptr(out), N.ptr(ws), nb, N.stream_ptr())
     assert close(S.snr_sq_device(sigs, rows, res), out)
+
+
+@pytest.mark.parametrize('n,longest', [(1025, 2), (1026, 64), (2600, 700), (3000, 65)])
+def test_ragged_order_changes_no_result(n, longest):
+    """A ragged batch taken longest first (a workspace with room for the order)
+    and as it comes (one of the records and counters alone): bit for bit the
+    same matrices, whatever the spread of the lengths."""
+    import torch
+    from tests._common import NET_C1, hip_net
+    from gwfast_amd import _engine as E, _native as N, signal as S
+    wf = _wf(11)
+    rows = E.to_dev(E.param_rows(_events(11, n, 2), False))
+    lengths = E.to_dev(np.random.default_rng(n).integers(2, longest + 1, n).astype(np.int32), torch.int32)
+    sigs = list(hip_net(wf, NET_C1, True).signals.values())
+    full = int(N.lib().gwf_workspace_bytes(n))
+    ws = torch.empty(full, dtype=torch.uint8, device='cuda')
+    out = []
+    for size in (full, full - 4 * n):
+        F = torch.full((11, 11, n), float('nan'), dtype=torch.float64, device='cuda')
+        E.call('gwf_fisher_ragged', wf.c_struct(), S._dets(sigs), len(sigs), N.ptr(rows), rows.stride(0), n,
+               N.ptr(lengths), -1, N.ptr(F), N.ptr(ws), size, N.stream_ptr())
+        out.append(F.cpu().numpy())
+    assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
