@@ -52,15 +52,31 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
   u += 0x7FFFu + ((u >> 16) & 1u);
   return (uint16_t)(u >> 16);
 }
-// z / (1 + exp(-z)): the quotient z * rcp(d) corrected once by its exact
-// remainder, which rounds as the division does without its scaling of large
-// and small denominators (1 <= d <= e^80 here).  Below z = -80 the result is
-// at most 2e-33 in size (the division's: -0); an infinite z gives NaN.
-__device__ __forceinline__ float silu(float z) {
-  const float d = 1.f + __expf(fminf(-z, 80.f));
+// z / (1 + exp(-z)) at |z| < SILU_CORE: the quotient z * rcp(d) corrected once
+// by its exact remainder, which rounds as the division does without its
+// scaling of large and small denominators (1 <= d <= e^80 here).
+constexpr float SILU_CORE = 80.f;
+__device__ __forceinline__ float silu_core(float z) {
+  const float d = 1.f + __expf(-z);
   const float r = __builtin_amdgcn_rcpf(d);
   const float q = z * r;
   return fmaf(fmaf(-d, q, z), r, q);
+}
+// The same at every z.  Past the core the division itself: above, it gives z
+// (+inf too); below, where d grows to infinity at -88.7, values down to -0;
+// -inf / inf is NaN.
+__device__ __forceinline__ float silu(float z) {
+  return fabsf(z) < SILU_CORE ? silu_core(z) : z / (1.f + __expf(-z));
+}
+// f(SiLU) for values of which a lane's largest modulus is zmax (NaN aside):
+// one test of the wave's, so that the division is paid for where it is needed
+// only.  f(g) applies g, element by element the same function either way.
+template <class F>
+__device__ __forceinline__ void with_silu(float zmax, F&& f) {
+  if (__builtin_expect(__any(zmax >= SILU_CORE), 0))
+    f([](float z) { return silu(z); });
+  else
+    f([](float z) { return silu_core(z); });
 }
 // two values to bf16, rounded to nearest even, a in the low half
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -394,22 +410,29 @@ __global__ __launch_bounds__(256, 1) void k_mlp_fwd(const uint16_t* __restrict__
     const float4 bias = *(const float4*)(wf + boff + col);
     const float bj[4] = {bias.x, bias.y, bias.z, bias.w};
     uint16_t* hs = Hs[l & 1];
+    float z[4][4], zmax = 0.f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 4 * q + r;
-      float z[4], h[4];
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        z[j] = acc[j][r] + bj[j];
-        h[j] = silu(z[j]);
+        z[r][j] = acc[j][r] + bj[j];
+        zmax = fmaxf(zmax, fabsf(z[r][j]));
       }
-      const uint2 hb = pack4(h);
-      *(uint2*)(hs + row * TR_LD + col) = hb;
-      if (m0 + row < M) {
-        *(float4*)(act.Z[l] + (m0 + row) * HID + col) = make_float4(z[0], z[1], z[2], z[3]);
-        *(uint2*)(act.H[l] + (m0 + row) * HID + col) = hb;
+    with_silu(zmax, [&](auto silu_of) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * q + r;
+        float h[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) h[j] = silu_of(z[r][j]);
+        const uint2 hb = pack4(h);
+        *(uint2*)(hs + row * TR_LD + col) = hb;
+        if (m0 + row < M) {
+          *(float4*)(act.Z[l] + (m0 + row) * HID + col) = make_float4(z[r][0], z[r][1], z[r][2], z[r][3]);
+          *(uint2*)(act.H[l] + (m0 + row) * HID + col) = hb;
+        }
       }
-    }
+    });
   };
   load_w(MlpParams::W2);
   __builtin_amdgcn_sched_barrier(0);
@@ -699,21 +722,36 @@ struct ScreenArgs {
 // stores to four rows.  The screen is bound by the VALU (the SiLU's 10
 // instructions for each of 768 activations, two of them quarter rate); with
 // this and the SiLU's shorter quotient 10^6 events take 454 us (591 TFLOP/s)
-// instead of 557, the predictions bit for bit the same.
-__device__ __forceinline__ void screen_epilogue(const f32x4 (&acc)[8][4], const float* __restrict__ bias, int wave,
-                                                int lane, uint16_t* H) {
+// instead of 557, the predictions bit for bit the same; with the division
+// behind one test of a lane's 128 values (with_silu) 445, tested per 32 460.
+__device__ __forceinline__ void screen_epilogue(f32x4 (&acc)[8][4], const float* __restrict__ bias, int wave, int lane,
+                                                uint16_t* H) {
+  float zmax = 0.f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int col = 64 * wave + 16 * j + 4 * (lane >> 4);
     const float bj[4] = {bias[col], bias[col + 1], bias[col + 2], bias[col + 3]};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float h[4];
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) h[r] = silu(acc[i][j][r] + bj[r]);
-      *(uint2*)(H + (16 * i + (lane & 15)) * SCR_LD + col) = make_uint2(f2bf2(h[0], h[1]), f2bf2(h[2], h[3]));
-    }
+      for (int r = 0; r < 4; ++r) {
+        acc[i][j][r] += bj[r];
+        zmax = fmaxf(zmax, fabsf(acc[i][j][r]));
+      }
   }
+  with_silu(zmax, [&](auto act) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int col = 64 * wave + 16 * j + 4 * (lane >> 4);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float h[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h[r] = act(acc[i][j][r]);
+        *(uint2*)(H + (16 * i + (lane & 15)) * SCR_LD + col) = make_uint2(f2bf2(h[0], h[1]), f2bf2(h[2], h[3]));
+      }
+    }
+  });
 }
 
 // one 256 -> 256 layer: acc = H W^T with H (128 x 256) in LDS, W (256 x 256)

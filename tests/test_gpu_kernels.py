@@ -263,3 +263,72 @@ def test_ragged_order_changes_no_result(n, longest):
                N.ptr(lengths), -1, N.ptr(F), N.ptr(ws), size, N.stream_ptr())
         out.append(F.cpu().numpy())
     assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
+
+
+# z and SiLU(z): past the exponential's overflow (-88.72) the quotient is -0, -inf / inf has no value
+SILU_EXTREMES = [(-3.0e38, -0.), (-1e30, -0.), (-1e10, -0.), (-1000., -0.), (-100., -0.), (0., 0.), (-0., -0.),
+                 (80., 80.), (1000., 1000.), (1e30, 1e30), (3.0e38, 3.0e38), (np.inf, np.inf), (-np.inf, np.nan),
+                 (np.nan, np.nan)]
+
+
+def test_silu_over_the_whole_range():
+    """gwf_bias_silu against z / (1 + exp(-z)) in FP64.  The result is a bf16
+    number (2^-8 of it covers its rounding and the FP32 exponential's error,
+    below 2^-16 at |z| < 89); past the exponential's overflow the quotient is
+    0, which is off by no more than 88.8 exp(-88.7) = 2.7e-37.  The extremes
+    exactly."""
+    import torch
+    from gwfast_amd import _engine as E, _native as N
+    z = np.concatenate([np.linspace(-95., 95., 4001), -np.geomspace(1e-6, 3e38, 1000), np.geomspace(1e-6, 3e38, 1000)])
+    ext = np.array(SILU_EXTREMES, dtype=np.float32)
+    zf = np.concatenate([z.astype(np.float32), ext[:, 0]])
+    C = torch.as_tensor(zf, device='cuda').contiguous()
+    zero = torch.zeros(1, dtype=torch.float32, device='cuda')
+    H = torch.empty(zf.size, dtype=torch.bfloat16, device='cuda')
+    E.call('gwf_bias_silu', N.ptr(C), N.ptr(zero), zf.size, 1, None, N.ptr(H), N.stream_ptr())
+    h = H.to(torch.float64).cpu().numpy()
+    z64 = zf[:z.size].astype(np.float64)
+    with np.errstate(over='ignore'):
+        ref = z64 / (1. + np.exp(-z64))
+    assert np.all(np.abs(h[:z.size] - ref) <= 2. ** -8 * np.abs(ref) + 2.7e-37)
+    want = torch.as_tensor(ext[:, 1]).to(torch.bfloat16).to(torch.float64).numpy()
+    assert np.array_equal(h[z.size:], want, equal_nan=True)
+
+
+@pytest.mark.parametrize('unit', [0, 63, 64, 255])
+def test_a_saturated_unit_is_the_same_in_training_and_screen(unit):
+    """One unit far below and far above the exponential's range in every
+    layer, and one of infinite activation: the screen's prediction, the
+    training forward's and, for the finite ones, 64-bit arithmetic on the same
+    bf16 weights (the saturated unit's SiLU is -0, or the unit itself) agree."""
+    import torch
+    from gwfast_amd import _engine as E, screen
+    n = 200
+    rows = E.to_dev(E.param_rows(catalog.draw_bbh(n, seed=4), False))
+    for bias, value in ((-1e30, 0.), (-3e38, 0.), (-90., 0.), (np.inf, np.inf)):
+        sc = screen.SNRScreen(seed=1)
+        sc.fit_normalisation(rows, torch.zeros(n, dtype=torch.float64))
+        theta = sc.params()
+        for b in ('b1', 'b2', 'b3'):
+            theta[screen.OFFSETS[b][0] + unit] = bias
+        if np.isinf(value):  # no products of the infinite unit but the output's
+            for b in ('b1', 'b2'):
+                theta[screen.OFFSETS[b][0] + unit] = 0.
+            theta[screen.OFFSETS['w4'][0] + unit] = 1.
+        sc.set_params(theta)
+        y = sc.forward_train(sc.features(rows))[0].to(torch.float64).cpu().numpy()
+        ls = sc.predict_log_snr(rows).to(torch.float64).cpu().numpy()
+        if np.isinf(value):
+            assert np.all(y == np.inf) and np.all(ls == np.inf) and int(sc.classify(rows).min()) == 2
+            continue
+        h = sc.features(rows).to(torch.float64).cpu().numpy()
+        f64 = lambda flat, name: sc._view(flat, name).to(torch.float64).cpu().numpy()
+        for l in '123':
+            zl = h @ f64(sc.theta_bf, 'W' + l).T + f64(sc.theta, 'b' + l)
+            with np.errstate(over='ignore'):
+                hl = zl / (1. + np.exp(-zl))
+            h = torch.as_tensor(hl).to(torch.bfloat16).to(torch.float64).numpy()
+        ref = h @ f64(sc.theta, 'w4') + f64(sc.theta, 'b4')
+        # activations differ by a bf16 rounding (2^-8) where FP32 and FP64 fall on two sides of a tie
+        tol = 2. ** -8 * 3 * (np.abs(h) @ np.abs(f64(sc.theta, 'w4')) + np.abs(ref))
+        assert np.all(np.abs(y - ref) <= tol) and np.all(np.abs(ls - y * sc.y_scale - sc.y_shift) <= tol)
