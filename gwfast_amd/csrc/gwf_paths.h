@@ -308,7 +308,10 @@ GWF_HD void setup_event_consts(const NetK& net, const double* par, int64_t ld, i
 // The part of the record that the SNR reads: the amplitude's coefficients and
 // fcut (values, in the same slots, without the phase's and every tangent,
 // whose arithmetic the compiler then drops) and the event's constants.  The
-// tau coefficients' tangents come from what the record held and are not read.
+// tangents of tau's coefficients and of the plus polarisation's inclination
+// factor, which only the Fisher kernels read, are NaN: a Fisher matrix of such
+// a record has a NaN row and column, where it would else be made of whatever
+// the record held before.
 template <int MODEL>
 GWF_HD void setup_event_snr(const gwf_waveform& w, const NetK& net, const double* par, int64_t ld, int64_t e,
                             double* rec) {
@@ -331,7 +334,10 @@ GWF_HD void setup_event_snr(const gwf_waveform& w, const NetK& net, const double
     rec[TF_FCUT * SLOT] = tf2_fcut(w, Mc, eta, chi1, chi2);
   }
   constexpr int MGS = is_pd(MODEL) ? (int)PD_MG : (int)TF_MG, FCS = is_pd(MODEL) ? (int)PD_FCUT : (int)TF_FCUT;
-  setup_event_consts(net, par, ld, e, rec + MGS * SLOT, rec[FCS * SLOT], rec);
+  const double nan = __builtin_nan("");
+  const double mg[3] = {rec[MGS * SLOT], nan, nan};
+  setup_event_consts(net, par, ld, e, mg, rec[FCS * SLOT], rec);
+  rec[REC_EV + EV_DCP] = nan;
 }
 
 // Fills the event record: waveform coefficients (duals) + projection constants.

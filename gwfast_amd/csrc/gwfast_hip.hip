@@ -221,8 +221,8 @@ __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const d
   }
 }
 
-// The SNR's records (setup_event_snr), one lane per event: values of the
-// amplitude's slots alone, where k_setup's tangents and phase bound a large
+// The records of gwf_snr_once (setup_event_snr), one lane per event: values of
+// the amplitude's slots alone, where k_setup's tangents and phase bound a large
 // batch (10^5 IMRPhenomD events: k_setup 310 us, this 81) and its chain a
 // small one (100 tidal TaylorF2 events 12 us, 7).
 template <int MODEL>
@@ -2821,9 +2821,8 @@ int launch_setup(const gwf_waveform* wf, const NetK& net, const double* par, int
   return hip_check(hipGetLastError(), "setup launch");
 }
 
-// The records of an SNR call on its own (launch_setup's where a caller
-// prepares them: they may go to the Fisher kernels).  One lane per event;
-// blocks as launch_setup's.
+// The records of gwf_snr_once (every other call's are launch_setup's: they may
+// go to the Fisher kernels).  One lane per event; blocks as launch_setup's.
 int launch_setup_snr(const gwf_waveform* wf, const NetK& net, const double* par, int64_t ld, int64_t n_ev,
                      double* rec, hipStream_t st) {
   const int bs = n_ev <= 65536 * 4 ? 64 : 256;
@@ -3175,9 +3174,18 @@ int gwf_fisher_arms(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_
 
 int gwf_snr(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, const double* params, int64_t ld,
             int64_t n_ev, int32_t res, double* snrsq_out, void* workspace, size_t ws_bytes, void* stream) {
-  int rc = prepare_impl(wf, dets, n_det, params, ld, n_ev, res, true, workspace, ws_bytes, stream);
+  int rc = gwf_prepare(wf, dets, n_det, params, ld, n_ev, res, workspace, ws_bytes, stream);
   if (rc) return rc;
   return gwf_snr_prepared(wf, dets, n_det, n_ev, res, snrsq_out, workspace, ws_bytes, stream);
+}
+
+int gwf_snr_once(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, const double* params, int64_t ld,
+                 int64_t n_ev, int32_t res, const int32_t* res_ev, double* snrsq_out, void* workspace, size_t ws_bytes,
+                 void* stream) {
+  if (res_ev) res = 2;  // not read
+  int rc = prepare_impl(wf, dets, n_det, params, ld, n_ev, res, true, workspace, ws_bytes, stream);
+  if (rc) return rc;
+  return snr_prepared_impl(wf, dets, n_det, n_ev, res, res_ev, snrsq_out, workspace, ws_bytes, stream);
 }
 
 int gwf_fisher(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, const double* params, int64_t ld,
@@ -3203,7 +3211,7 @@ int gwf_snr_ragged(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_d
                    int64_t n_ev, const int32_t* res_ev, double* snrsq_out, void* workspace, size_t ws_bytes,
                    void* stream) {
   if (n_ev > 0 && !res_ev) return fail(-EINVAL, "res_ev is NULL");
-  int rc = prepare_impl(wf, dets, n_det, params, ld, n_ev, 2, true, workspace, ws_bytes, stream);
+  int rc = gwf_prepare(wf, dets, n_det, params, ld, n_ev, 2, workspace, ws_bytes, stream);
   if (rc) return rc;
   return snr_prepared_impl(wf, dets, n_det, n_ev, 2, res_ev, snrsq_out, workspace, ws_bytes, stream);
 }

@@ -417,12 +417,8 @@ def snr_sq_device(signals, rows, res):
     out = t.empty((narms, n), dtype=t.float64, device=rows.device)
     ws, nb = E.workspace(n)
     r, r_ev = _res_arg(res, n, rows.device)
-    if r_ev is None:
-        E.call('gwf_snr', wf.c_struct(), _dets(signals), len(signals), N.ptr(rows), rows.stride(0), n, r, N.ptr(out),
-               N.ptr(ws), nb, N.stream_ptr())
-    else:
-        E.call('gwf_snr_ragged', wf.c_struct(), _dets(signals), len(signals), N.ptr(rows), rows.stride(0), n,
-               N.ptr(r_ev), N.ptr(out), N.ptr(ws), nb, N.stream_ptr())
+    E.call('gwf_snr_once', wf.c_struct(), _dets(signals), len(signals), N.ptr(rows), rows.stride(0), n,
+           r if r_ev is None else 2, N.ptr(r_ev), N.ptr(out), N.ptr(ws), nb, N.stream_ptr())
     return out
 
 

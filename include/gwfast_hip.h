@@ -190,11 +190,20 @@ int gwf_fisher_ragged(const gwf_waveform* wf, const gwf_detector* dets, int32_t 
                       int64_t n_ev, const int32_t* res_ev, int32_t arm, double* fisher_out, void* workspace,
                       size_t ws_bytes, void* stream);
 
+/* gwf_snr (res_ev NULL) and gwf_snr_ragged (res_ev given; res unused) for
+ * callers who want the SNRs alone: the workspace is left with the values the
+ * SNR reads and nothing else, at about a quarter of the setup's time.  Such
+ * records serve gwf_snr_prepared only; a Fisher matrix of them has NaN in it. */
+int gwf_snr_once(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, const double* params, int64_t ld,
+                 int64_t n_ev, int32_t res, const int32_t* res_ev, double* snrsq_out, void* workspace, size_t ws_bytes,
+                 void* stream);
+
 /* The two halves of gwf_snr / gwf_fisher, for callers that reuse the
  * per-event records (e.g. SNR then Fisher of the same events) or time the
  * integral kernels alone.  gwf_prepare fills the workspace with the event
- * records of a (waveform, network, res) triple; the *_prepared calls must be
- * given the same triple and workspace. */
+ * records of a (waveform, network, res) triple, as gwf_snr, gwf_fisher and
+ * their ragged forms leave them too; the *_prepared calls must be given the
+ * same triple and workspace. */
 int gwf_prepare(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, const double* params, int64_t ld,
                 int64_t n_ev, int32_t res, void* workspace, size_t ws_bytes, void* stream);
 int gwf_snr_prepared(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, int64_t n_ev, int32_t res,

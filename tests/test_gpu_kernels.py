@@ -332,3 +332,79 @@ def test_a_saturated_unit_is_the_same_in_training_and_screen(unit):
         # activations differ by a bf16 rounding (2^-8) where FP32 and FP64 fall on two sides of a tie
         tol = 2. ** -8 * 3 * (np.abs(h) @ np.abs(f64(sc.theta, 'w4')) + np.abs(ref))
         assert np.all(np.abs(y - ref) <= tol) and np.all(np.abs(ls - y * sc.y_scale - sc.y_shift) <= tol)
+
+
+def _models():
+    from gwfast_amd.waveforms import IMRPhenomD_NRTidalv2
+    return {11: lambda: _wf(11), 12: lambda: _wf(12), 13: lambda: _wf(13), 14: lambda: _wf(14),
+            'NRTidalv2': lambda: IMRPhenomD_NRTidalv2()}
+
+
+def _model_rows(P, n, seed):
+    from gwfast_amd import _engine as E
+    tidal = P in (13, 14, 'NRTidalv2')
+    ev = _events(14 if P == 14 else (13 if tidal else P), n, seed)
+    return E.to_dev(E.param_rows(ev, tidal, P in (12, 14)))
+
+
+@pytest.mark.parametrize('P', [11, 12, 13, 14, 'NRTidalv2'])
+@pytest.mark.parametrize('n', [1, 3, 300])
+def test_snr_call_leaves_the_prepared_records(P, n):
+    """gwf_snr and gwf_snr_ragged are gwf_prepare and the SNR of its records:
+    the same SNR bit for bit, and a workspace (of NaN before) from which
+    gwf_fisher_prepared gives gwf_fisher's matrices bit for bit."""
+    import torch
+    from tests._common import NET_C1, hip_net
+    from gwfast_amd import _engine as E, _native as N, signal as S
+    wf, rows, res = _models()[P](), _model_rows(P, n, 8), 130
+    sigs = list(hip_net(wf, NET_C1, True).signals.values())
+    dets, nd, s = S._dets(sigs), len(sigs), N.stream_ptr()
+    nb = int(N.lib().gwf_workspace_bytes(n))
+    lengths = torch.full((n,), res, dtype=torch.int32, device='cuda')
+    F = S.fisher_device(sigs, wf, rows, res)
+
+    def workspace():
+        return torch.full((nb,), 0xff, dtype=torch.uint8, device='cuda')
+
+    def prepared(ws, entry, extra=()):
+        out = torch.empty(F.shape if entry == 'gwf_fisher_prepared' else (5, n), dtype=torch.float64, device='cuda')
+        E.call(entry, wf.c_struct(), dets, nd, n, res, *extra, N.ptr(out), N.ptr(ws), nb, s)
+        return out
+
+    ws = workspace()
+    E.call('gwf_prepare', wf.c_struct(), dets, nd, N.ptr(rows), rows.stride(0), n, res, N.ptr(ws), nb, s)
+    snr = prepared(ws, 'gwf_snr_prepared')
+    for entry, length in (('gwf_snr', res), ('gwf_snr_ragged', N.ptr(lengths))):
+        ws, out = workspace(), torch.empty((5, n), dtype=torch.float64, device='cuda')
+        E.call(entry, wf.c_struct(), dets, nd, N.ptr(rows), rows.stride(0), n, length, N.ptr(out), N.ptr(ws), nb, s)
+        assert torch.equal(out, snr)
+        assert torch.equal(prepared(ws, 'gwf_fisher_prepared', (-1,)), F)
+
+
+@pytest.mark.parametrize('P', [11, 12, 13, 14, 'NRTidalv2'])
+@pytest.mark.parametrize('motion', [True, False])
+def test_records_of_the_snr_alone_give_no_fisher_matrix(P, motion):
+    """gwf_snr_once's records: gwf_snr_prepared reads them like any, and the
+    Fisher matrix of every event has NaN in it, whatever the records held
+    before (those of gwf_prepare here), for network sums and single arms."""
+    import torch
+    from tests._common import NET_C1, hip_net
+    from gwfast_amd import _engine as E, _native as N, signal as S
+    wf, n, res = _models()[P](), 5, 130
+    rows = _model_rows(P, n, 8)
+    sigs = list(hip_net(wf, NET_C1, motion).signals.values())
+    dets, nd, s = S._dets(sigs), len(sigs), N.stream_ptr()
+    nb = int(N.lib().gwf_workspace_bytes(n))
+    ws = torch.empty(nb, dtype=torch.uint8, device='cuda')
+    for lengths in (None, torch.full((n,), res, dtype=torch.int32, device='cuda')):
+        E.call('gwf_prepare', wf.c_struct(), dets, nd, N.ptr(rows), rows.stride(0), n, res, N.ptr(ws), nb, s)
+        out, again = torch.empty((2, 5, n), dtype=torch.float64, device='cuda')
+        E.call('gwf_snr_once', wf.c_struct(), dets, nd, N.ptr(rows), rows.stride(0), n, res, N.ptr(lengths),
+               N.ptr(out), N.ptr(ws), nb, s)
+        E.call('gwf_snr_prepared', wf.c_struct(), dets, nd, n, res, N.ptr(again), N.ptr(ws), nb, s)
+        assert bool((out > 0).all()) and torch.equal(out, again)
+        for arm in (-1, 0, 4):
+            F = torch.empty((wf.nParams, wf.nParams, n), dtype=torch.float64, device='cuda')
+            E.call('gwf_fisher_prepared', wf.c_struct(), dets, nd, n, res, arm, N.ptr(F), N.ptr(ws), nb, s)
+            assert bool(torch.isnan(F[5]).all()) and bool(torch.isnan(F[:, 5]).all())
+    assert S.snr_sq_device(sigs, rows[:, :0].contiguous(), np.zeros(0, dtype=np.int32)).shape == (5, 0)
