@@ -1329,8 +1329,10 @@ __global__ __launch_bounds__(256, 3) void k_snr(gwf_waveform w, NetK net, const 
 // A block of SNR_WAVES waves per event, for batches that would leave SIMDs
 // without a wave: wave q takes chunk q of every SNR_WAVES, its points' weights
 // and |h|^2 go to LDS, and wave k adds arm k's in chunk order, as k_snr does
-// (the same sums in the same order).  Up to MAXA = 8 arms: the LDS holds 64 KB
-// of them.  100 tidal TaylorF2 events x 1000 points, three arms: 34 us with a
+// (the same sums in the same order, and the same bits: the compiler contracts
+// snr_points alike in both kernels, which a test holds it to, so that an
+// event's SNR does not depend on its batch).  Up to MAXA = 8 arms: the LDS
+// holds 64 KB of them.  100 tidal TaylorF2 events x 1000 points, three arms: 34 us with a
 // wave per event (16 chunks one after another), 18 us with a block.
 constexpr int SNR_WAVES = 8;
 template <int MODEL>

@@ -408,3 +408,27 @@ def test_records_of_the_snr_alone_give_no_fisher_matrix(P, motion):
             E.call('gwf_fisher_prepared', wf.c_struct(), dets, nd, n, res, arm, N.ptr(F), N.ptr(ws), nb, s)
             assert bool(torch.isnan(F[5]).all()) and bool(torch.isnan(F[:, 5]).all())
     assert S.snr_sq_device(sigs, rows[:, :0].contiguous(), np.zeros(0, dtype=np.int32)).shape == (5, 0)
+
+
+@pytest.mark.parametrize('P', [11, 12, 13, 14, 'NRTidalv2'])
+@pytest.mark.parametrize('sites', [1, 2, 3, 4, 6])
+@pytest.mark.parametrize('res', [2, 63, 65, 513, 1000])
+def test_snr_does_not_depend_on_the_batch(P, sites, res):
+    """An event's SNR alone, among a few and among many (uniform and ragged
+    grids): bit for bit, so that a catalogue in chunks of any size, or resumed
+    in others, holds the same SNRs."""
+    import torch
+    from tests._common import hip_net
+    from gwfast_amd import gwfastGlobals as glob, signal as S
+    wf, n = _models()[P](), 7
+    rows = _model_rows(P, n, 8)
+    net = [(s, glob.PSD_ET if s[0] == 'E' else glob.PSD_CE) for s in ['CE1Id', 'ETS', 'CE2NM', 'Virgo', 'KAGRA', 'ETMR'][:sites]]
+    sigs = list(hip_net(wf, net, True).signals.values())
+    lengths = np.array([res, 2, 64, max(2, res // 2), res, 700, 129], dtype=np.int32)
+    for ln in (res, lengths):
+        pick = lambda i: ln if np.isscalar(ln) else ln[i:i + 1]
+        many = S.snr_sq_device(sigs, rows.repeat(1, 200).contiguous(), ln if np.isscalar(ln) else np.tile(ln, 200))
+        assert torch.equal(many, many[:, :n].repeat(1, 200))
+        assert torch.equal(S.snr_sq_device(sigs, rows, ln), many[:, :n])
+        for i in range(2):
+            assert torch.equal(S.snr_sq_device(sigs, rows[:, i:i + 1].contiguous(), pick(i)), many[:, i:i + 1])
