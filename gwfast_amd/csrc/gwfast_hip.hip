@@ -1025,6 +1025,7 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
 #endif
   if (wave < PC_EPB) {
     int k = 0;  // items produced by this pair
+    const bool ordered = RAGGED && order && __builtin_amdgcn_readfirstlane((int)counter[2]) != 0;  // k_ragged_order
     int64_t e = RAGGED ? 0 : (int64_t)blockIdx.x * PC_EPB + slot;
     const int64_t stride = (int64_t)gridDim.x * PC_EPB;
     for (;;) {
@@ -1032,7 +1033,7 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
         unsigned int t0 = 0;
         if (lane == 0) t0 = atomicAdd(counter, 1u);
         e = (int64_t)__builtin_amdgcn_readfirstlane((int)__shfl(t0, 0, 64));
-        if (order && e < n_ev) e = (int64_t)__builtin_amdgcn_readfirstlane((int)order[e]);
+        if (ordered && e < n_ev) e = (int64_t)__builtin_amdgcn_readfirstlane((int)order[e]);
       }
       const int s0 = k % NB;
       if (e >= n_ev) {  // end marker
@@ -1202,25 +1203,88 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
 // The events of a ragged batch by falling number of 64-point chunks (within a
 // 1024th of the largest; events of one such class in any order), for the
 // event queue: taken as they come, the pairs' last events end up to a
-// longest event apart (2 x 10^4 tidal TaylorF2 events of 500 to 10^4 points:
-// 7.35 ms, in this order 7.09 with the 30 us of this kernel).  One block;
-// three passes over the lengths.
+// longest event apart.  One block; clears the queue counters (counter[0],
+// counter[1]) and says in counter[2] whether there is an order.
+// What the order saves grows with the spread of the lengths (some 2 us per
+// chunk of it, once per batch); what it costs grows with n_ev: the sort 10 us
+// at 2 x 10^4, and neighbouring events' results no longer written together.
+// Measured on IMRPhenomD events in five arms, as they come and ordered, the
+// spread in chunks against the line:
+//   2 x 10^4 events, 500..10^4 points  149 : 17   6411 -> 6095 us
+//   2 x 10^4 events, 64..2000 points    31 : 17   1435 -> 1409
+//   2 x 10^3 events, 50..1000 points    15 :  8    156 ->  128
+//   10^5 events, 500..10^4 points      149 : 56  30428 -> 30227
+//   5 x 10^4 events, 64..2000 points    31 : 32   3437 -> 3437 (left as they come)
+// A batch left as it comes pays 2-4 us for the look at its lengths (10^5 of
+// 65..256 points 1950 -> 1953 us; sorted by a slower form of this 2091).
+constexpr int ORDER_AHEAD = 8;       // lengths a thread has in flight
+constexpr int ORDER_SAMPLE = 4096;   // lengths that the spread is taken from, at least
+__device__ __forceinline__ bool order_pays(int spread, int64_t n_ev) { return spread > 8 + n_ev / 2048; }
+
 __global__ __launch_bounds__(1024) void k_ragged_order(const int* __restrict__ res_ev, int64_t n_ev,
+                                                       unsigned int* __restrict__ counter,
                                                        uint32_t* __restrict__ order) {
   __shared__ unsigned int first[1024], scan[1024];
-  __shared__ int longest;
-  const int tid = threadIdx.x;
-  auto chunks = [&](int64_t i) { return (min(max(res_ev[i], 2), 1 << 30) + 63) / 64; };
-  if (tid == 0) longest = 0;
+  __shared__ int longest, shortest;
+  const int tid = threadIdx.x, lane = tid & 63;
+  // f(i, chunks of i) for every step-th group of 64 neighbouring events
+  auto each = [&](int64_t step, auto f) {
+    const int64_t next = 1024 * step;  // a wave's next group
+    for (int64_t i0 = (tid - lane) * step + lane; i0 < n_ev; i0 += ORDER_AHEAD * next) {
+      int r[ORDER_AHEAD];
+#pragma unroll
+      for (int k = 0; k < ORDER_AHEAD; ++k) {
+        const int64_t i = i0 + k * next;
+        r[k] = i < n_ev ? res_ev[i] : 0;
+      }
+#pragma unroll
+      for (int k = 0; k < ORDER_AHEAD; ++k) {
+        const int64_t i = i0 + k * next;
+        if (i < n_ev) f(i, (min(max(r[k], 2), 1 << 30) + 63) / 64);
+      }
+    }
+  };
+  if (tid == 0) {
+    longest = 0;
+    shortest = 1 << 30;
+  }
+  if (tid < 2) counter[tid] = 0u;
   first[tid] = 0;
   __syncthreads();
-  int m = 0;
-  for (int64_t i = tid; i < n_ev; i += 1024) m = max(m, chunks(i));
-  atomicMax(&longest, m);
+  {
+    int lo = 1 << 30, hi = 0;
+    each(max(n_ev / ORDER_SAMPLE, (int64_t)1), [&](int64_t, int c) {
+      lo = min(lo, c);
+      hi = max(hi, c);
+    });
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = min(lo, __shfl_xor(lo, o));
+      hi = max(hi, __shfl_xor(hi, o));
+    }
+    if (lane == 0) {
+      atomicMin(&shortest, lo);
+      atomicMax(&longest, hi);
+    }
+  }
   __syncthreads();
+  const bool pays = order_pays(longest - shortest, n_ev);
+  if (tid == 0) counter[2] = pays ? 1u : 0u;
+  if (!pays) return;
   const int64_t div = (int64_t)longest + 1;
-  auto bin = [&](int64_t i) { return 1023 - (int)((int64_t)chunks(i) * 1024 / div); };
-  for (int64_t i = tid; i < n_ev; i += 1024) atomicAdd(&first[bin(i)], 1u);
+  auto bin = [&](int c) { return 1023 - (int)((int64_t)min(c, longest) * 1024 / div); };  // 0: longer than the sample's
+  // adds 1 to the class of every live lane and gives the number before it; the
+  // lanes of the first lane's class by one atomic (most events may share a few)
+  auto add = [&](int b) {
+    const int b0 = __builtin_amdgcn_readfirstlane(b);
+    const uint64_t same = __ballot(b == b0);
+    if (b != b0) return atomicAdd(&first[b], 1u);
+    const unsigned int below = (unsigned int)__popcll(same & ((1ull << lane) - 1));
+    unsigned int n0 = 0;
+    if (below == 0) n0 = atomicAdd(&first[b0], (unsigned int)__popcll(same));
+    return (unsigned int)__builtin_amdgcn_readfirstlane((int)n0) + below;  // the first lane of `same` is below == 0
+  };
+  each(1, [&](int64_t, int c) { add(bin(c)); });
   __syncthreads();
   // exclusive prefix sum of the classes' sizes
   scan[tid] = first[tid];
@@ -1233,7 +1297,7 @@ __global__ __launch_bounds__(1024) void k_ragged_order(const int* __restrict__ r
   }
   first[tid] = scan[tid] - first[tid];
   __syncthreads();
-  for (int64_t i = tid; i < n_ev; i += 1024) order[atomicAdd(&first[bin(i)], 1u)] = (uint32_t)i;
+  each(1, [&](int64_t i, int c) { order[add(bin(c))] = (uint32_t)i; });
 }
 
 // After k_fisher_pq: NaN in every output element when a wave's wait ran out.
@@ -2745,7 +2809,7 @@ int cu_count(int* n_cu) {
 
 // The network Fisher on producer / consumer pairs (k_fisher_pq): one
 // resident block per CU, then the NaN fill that reports an expired wait.
-// counter: two words, zeroed here.  order: n_ev words for a ragged batch's
+// counter: three words, set here.  order: n_ev words for a ragged batch's
 // order, or NULL.
 template <bool LIN, bool RAGGED, int MODE = PQ_SUM>
 int launch_fisher_pq(const gwf_waveform* wf, hipStream_t st, const NetK& net_in, const double* rec, int64_t n_ev,
@@ -2754,10 +2818,12 @@ int launch_fisher_pq(const gwf_waveform* wf, hipStream_t st, const NetK& net_in,
   int n_cu = 0;
   int rc = cu_count(&n_cu);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, counter, 2);
   const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((n_ev + PC_EPB - 1) / PC_EPB, n_cu));
   if (n_ev <= blocks * PC_EPB) order = nullptr;  // no queue
-  if (RAGGED && order) hipLaunchKernelGGL(k_ragged_order, dim3(1), dim3(1024), 0, st, res_ev, n_ev, order);
+  if (RAGGED && order)
+    hipLaunchKernelGGL(k_ragged_order, dim3(1), dim3(1024), 0, st, res_ev, n_ev, counter, order);
+  else
+    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, counter, 2);
   NetK net = net_in;
   net.spin_limit = g_pq_spin_limit;
   const dim3 g((unsigned)blocks), b(128 * PC_EPB);

@@ -432,3 +432,45 @@ def test_snr_does_not_depend_on_the_batch(P, sites, res):
         assert torch.equal(S.snr_sq_device(sigs, rows, ln), many[:, :n])
         for i in range(2):
             assert torch.equal(S.snr_sq_device(sigs, rows[:, i:i + 1].contiguous(), pick(i)), many[:, i:i + 1])
+
+
+@pytest.mark.parametrize('n', [1025, 1500, 4096, 9001, 20011])
+@pytest.mark.parametrize('kind', ['equal', 'narrow', 'wide', 'few long', 'longest unseen', 'out of range'])
+def test_ragged_order_where_it_pays_and_where_not(n, kind):
+    """The order is made by the spread of a sample of the lengths (every
+    n // 4096-th group of 64): with it, without (a workspace of the records and
+    counters alone) and for events by themselves the same matrices bit for bit,
+    with the longest events in the sample or not and lengths below 2 (taken as
+    2)."""
+    import torch
+    from tests._common import NET_C1, hip_net
+    from gwfast_amd import _engine as E, _native as N, signal as S
+    wf = _wf(11)
+    rows = E.to_dev(E.param_rows(_events(11, 500, 2), False)).repeat(1, n // 500 + 1)[:, :n].contiguous()
+    rng = np.random.default_rng(n)
+    lengths = rng.integers(2, 130, n)
+    if kind == 'equal':
+        lengths[:] = 64
+    elif kind == 'wide':
+        lengths = rng.integers(2, 1500, n)
+    elif kind == 'few long':
+        lengths[rng.random(n) < 0.01] = 2000
+    elif kind == 'longest unseen':
+        lengths[::64] = 1500
+        lengths[65:128] = 4000
+    elif kind == 'out of range':
+        lengths[::7], lengths[1::7], lengths[-1] = -5, 0, 1400
+    sigs = list(hip_net(wf, NET_C1, True).signals.values())
+    full = int(N.lib().gwf_workspace_bytes(n))
+    ws = torch.full((full,), 0xff, dtype=torch.uint8, device='cuda')
+    L = E.to_dev(lengths.astype(np.int32), torch.int32)
+    out = []
+    for size in (full, full - 4 * n):
+        F = torch.full((11, 11, n), float('nan'), dtype=torch.float64, device='cuda')
+        E.call('gwf_fisher_ragged', wf.c_struct(), S._dets(sigs), len(sigs), N.ptr(rows), rows.stride(0), n,
+               N.ptr(L), -1, N.ptr(F), N.ptr(ws), size, N.stream_ptr())
+        out.append(F)
+    assert bool(torch.isfinite(out[0]).all()) and torch.equal(out[0], out[1])
+    for e in (0, 1, 66, n - 1):
+        one = S.fisher_device(sigs, wf, rows[:, e:e + 1].contiguous(), np.array([max(2, lengths[e])]))
+        assert torch.equal(out[0][:, :, e], one[:, :, 0])
