@@ -15,6 +15,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <utility>
 
 #include "gwf_paths.h"
 #include "gwf_net.h"
@@ -67,22 +68,30 @@ struct WaveSums {
   static constexpr int m(int s) { return (N + (1 << s) - 1) >> s; }
   static constexpr int R = m(6);
   double v[N];
+  // value J of step S; a few in flight: all at once, the values sent and kept
+  // would spill
+  template <int S, int J>
+  __device__ __forceinline__ void value(bool up) {
+    constexpr int off = 32 >> S, M = m(S), H = m(S + 1);
+    if constexpr (J + H < M) {
+      const double keep = up ? v[J + H] : v[J], send = up ? v[J] : v[J + H];
+      v[J] = keep + __shfl_xor(send, off, 64);
+    } else {
+      v[J] += __shfl_xor(v[J], off, 64);
+    }
+    if constexpr (J % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+  }
+  // (a fold, not a loop over J: at some N (49, 56, 58, 105) the compiler left one
+  // of the loops rolled and with it v in scratch memory: the 14-parameter Gram
+  // of 5000 events x 1000 points 561 us, 375 so)
+  template <int S, int... J>
+  __device__ __forceinline__ void values(bool up, std::integer_sequence<int, J...>) {
+    (value<S, J>(up), ...);
+  }
   template <int S>
   __device__ __forceinline__ void step(int lane) {
     if constexpr (S < 6) {
-      constexpr int off = 32 >> S, M = m(S), H = m(S + 1);
-      const bool up = (lane & off) != 0;
-#pragma unroll
-      for (int j = 0; j < H; ++j) {
-        if (j + H < M) {
-          const double keep = up ? v[j + H] : v[j], send = up ? v[j] : v[j + H];
-          v[j] = keep + __shfl_xor(send, off, 64);
-        } else {
-          v[j] += __shfl_xor(v[j], off, 64);
-        }
-        // a few in flight: all at once, the values sent and kept would spill
-        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-      }
+      values<S>((lane & (32 >> S)) != 0, std::make_integer_sequence<int, m(S + 1)>());
       step<S + 1>(lane);
     }
   }

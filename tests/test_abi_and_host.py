@@ -274,3 +274,22 @@ def test_any_arm_rotation_is_a_turned_x_arm():
         sig._psd_dev = tuple(type('T', (), {'data_ptr': lambda self: 0})() for _ in range(2))
         det = rot_detector(sig, 37.)
         assert det.xax_deg == pytest.approx(d['xax'] + 37.) and det.compute2arms == 0
+
+
+def test_sums_stay_in_registers(so_path):
+    """The built kernels' scratch memory (their metadata): none in the Gram
+    kernels, at most a few spilled registers in the producer / consumer Fisher
+    kernels (whose per-event sums are 450 to 860 bytes a lane), and no kernel
+    with a stack of unknown size."""
+    b = open(so_path, 'rb').read()
+    kernels = {}
+    for m in re.finditer(rb'(_ZN\w+?)\xbb\.private_segment_fixed_size(\xce.{4}|\xcd.{2}|\xcc.|[\x00-\x7f])', b, re.S):
+        v = m.group(2)
+        kernels[m.group(1).decode()] = int.from_bytes(v[1:], 'big') if len(v) > 1 else v[0]
+    gram = {k: v for k, v in kernels.items() if 'k_gramI' in k}
+    pairs = {k: v for k, v in kernels.items() if 'k_fisher_pqI' in k}
+    assert len(gram) == 4 and len(pairs) >= 30
+    assert set(gram.values()) == {0}
+    assert max(pairs.values()) <= 128, {k: v for k, v in pairs.items() if v > 128}
+    flags = re.findall(rb'\.uses_dynamic_stack(.)', b, re.S)
+    assert len(flags) >= len(kernels) and set(flags) == {b'\xc2'}
