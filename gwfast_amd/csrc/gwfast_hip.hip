@@ -200,34 +200,40 @@ __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const d
                                                int64_t n_ev, bool own_grid, double* __restrict__ rec) {
   // IMRPhenomD models: NT lanes per event, lane tk evaluating tangent tk
   // (setup_waveform_split), and grid row y the phase's coefficients, the
-  // amplitude's or the event's constants: three chains of about the same
-  // length, which as one bound every batch that does not fill the chip
-  // (IMRPhenomD, one chain and three: 1 to 1000 events 31 and 19 us, 10^4 42
-  // and 37, 3 x 10^4 87 and 93, 10^5 330 and 315; the same split at every
-  // size, so that a record does not depend on the batch).  TaylorF2: one lane
-  // per event
+  // amplitude's or (one lane per event) the event's constants: three chains of
+  // about the same length, which as one bound every batch that does not fill
+  // the chip (IMRPhenomD, one chain and three: 1 to 1000 events 32 and 19 us,
+  // 10^4 40 and 31, 3 x 10^4 81 and 78, 10^5 328 and 290; NRTidalv2 39 and 25,
+  // 48.7 and 48.1, 132 and 126, 449 and 406; the same split at every size, so
+  // that a record does not depend on the batch).  TaylorF2: one lane per event
   constexpr int LPE = is_pd(MODEL) ? NT : 1;
   const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if constexpr (is_pd(MODEL)) {
+    if (blockIdx.y == 2) {  // the constants: one lane per event
+      if (tid < n_ev) setup_pd_consts<MODEL>(net, par, ld, tid, rec + tid * (int64_t)REC_DOUBLES);
+      return;
+    }
+  }
   const int64_t e = tid / LPE;
   const int tk = (int)(tid - e * LPE);
   if (e >= n_ev) return;
+  double* r = rec + e * (int64_t)REC_DOUBLES;
+  if constexpr (is_pd(MODEL)) {
+    if (blockIdx.y == 1) {  // the amplitude, which has no reference frequency
+      setup_waveform_split<MODEL, PD_AMP>(w, par, ld, e, 1.0, r, tk);
+      return;
+    }
+  }
   double f0;
   if (own_grid) {  // minimum of the caller's grid column (waveforms.py:1139), from k_grid_min
-    f0 = rec[e * (int64_t)REC_DOUBLES + REC_F0];
+    f0 = r[REC_F0];
   } else {  // first grid point: 10**log10(fmin) for geomspace, fmin for linspace
     f0 = net.lin ? net.fmin : grid_f(log10(net.fmin), log10(net.fmin), 0, 1);
   }
-  double* r = rec + e * (int64_t)REC_DOUBLES;
-  if constexpr (is_pd(MODEL)) {
-    if (blockIdx.y == 0)
-      setup_waveform_split<MODEL, PD_PHASE>(w, par, ld, e, f0, r, tk);
-    else if (blockIdx.y == 1)
-      setup_waveform_split<MODEL, PD_AMP>(w, par, ld, e, f0, r, tk);
-    else if (tk == 0)
-      setup_pd_consts<MODEL>(net, par, ld, e, r);
-  } else {
+  if constexpr (is_pd(MODEL))
+    setup_waveform_split<MODEL, PD_PHASE>(w, par, ld, e, f0, r, tk);
+  else
     setup_event<MODEL, NT>(w, net, par, ld, e, f0, r);
-  }
 }
 
 // The records of gwf_snr_once (setup_event_snr), one lane per event: values of
@@ -2879,24 +2885,21 @@ int launch_setup(const gwf_waveform* wf, const NetK& net, const double* par, int
     const int eb = n_ev >= 16 ? 16 : (n_ev >= 4 ? 4 : 1);
     hipLaunchKernelGGL(k_grid_min, dim3((unsigned)((n_ev + eb - 1) / eb)), dim3(1024), 0, st, fgrid, n_ev, nf, eb, rec);
   }
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid, rec);
+  };
   if (wf->model == GWF_MODEL_IMRPHENOMD)
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_IMRPHENOMD, 4>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
-                       rec);
+    go(k_setup<GWF_MODEL_IMRPHENOMD, 4>);
   else if (wf->model == GWF_MODEL_IMRPHENOMD_NRTIDALV2)
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_IMRPHENOMD_NRTIDALV2, 6>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
-                       rec);
+    go(k_setup<GWF_MODEL_IMRPHENOMD_NRTIDALV2, 6>);
   else if (nt_of(wf) == 5)
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 5>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
-                       rec);
+    go(k_setup<GWF_MODEL_TAYLORF2, 5>);
   else if (nt_of(wf) == 7)  // tidal and eccentric TaylorF2, 14 parameters
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 7>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
-                       rec);
+    go(k_setup<GWF_MODEL_TAYLORF2, 7>);
   else if (nt_of(wf) == 6)
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 6>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
-                       rec);
+    go(k_setup<GWF_MODEL_TAYLORF2, 6>);
   else
-    hipLaunchKernelGGL((k_setup<GWF_MODEL_TAYLORF2, 4>), grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid,
-                       rec);
+    go(k_setup<GWF_MODEL_TAYLORF2, 4>);
   return hip_check(hipGetLastError(), "setup launch");
 }
 
@@ -3122,7 +3125,9 @@ static int snr_prepared_impl(const gwf_waveform* wf, const gwf_detector* dets, i
   if (n_ev == 0) return 0;
   if (!snrsq_out) return fail(-EINVAL, "snrsq_out is NULL");
   hipStream_t st = (hipStream_t)stream;
-  // no more events than CUs: a block of eight waves for each
+  // No more events than CUs: a block of eight waves for each, which no grid
+  // length makes slower (256 events, five arms, a wave and a block per event,
+  // launch included: 64 points 10 and 9 us, 128 13 and 9, 1000 50 and 19)
   const bool small = net.n_arms <= 8;  // per-arm accumulators held in registers
   int n_cu = 0;
   rc = cu_count(&n_cu);
