@@ -195,9 +195,18 @@ __global__ __launch_bounds__(1024) void k_grid_min(const double* __restrict__ f,
   if (ty == 0 && e < n_ev) rec[e * (int64_t)REC_DOUBLES + REC_F0] = red[tx];
 }
 
+// Grids of up to this many points are looked through by the setup's lanes
+// themselves, the IMRPhenomD models' NT lanes per event and eccentric
+// TaylorF2's one: there a launch costs more than the loads (the whole waveform
+// call with k_grid_min and with the loop: 10^5 eccentric events x 1 point 120
+// and 95 us, one event x 9 points 16.9 and 14.6; one IMRPhenomD event x 8
+// points 25.8 and 22.1).
+constexpr int64_t GRID_MIN_LOOP_PD = 12, GRID_MIN_LOOP_TF = 24;
+
 template <int MODEL, int NT>
 __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const double* __restrict__ par, int64_t ld,
-                                               int64_t n_ev, bool own_grid, double* __restrict__ rec) {
+                                               int64_t n_ev, bool own_grid, const double* __restrict__ fgrid,
+                                               int64_t nf, double* __restrict__ rec) {
   // IMRPhenomD models: NT lanes per event, lane tk evaluating tangent tk
   // (setup_waveform_split), and grid row y the phase's coefficients, the
   // amplitude's or (one lane per event) the event's constants: three chains of
@@ -225,7 +234,10 @@ __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const d
     }
   }
   double f0;
-  if (own_grid) {  // minimum of the caller's grid column (waveforms.py:1139), from k_grid_min
+  if (fgrid) {  // minimum of the caller's grid column (waveforms.py:1139)
+    f0 = fgrid[e];
+    for (int64_t i = 1; i < nf; ++i) f0 = fmin(f0, fgrid[i * n_ev + e]);
+  } else if (own_grid) {  // the same from k_grid_min
     f0 = r[REC_F0];
   } else {  // first grid point: 10**log10(fmin) for geomspace, fmin for linspace
     f0 = net.lin ? net.fmin : grid_f(log10(net.fmin), log10(net.fmin), 0, 1);
@@ -2881,12 +2893,15 @@ int launch_setup(const gwf_waveform* wf, const NetK& net, const double* par, int
   const dim3 grid((unsigned)((nt + bs - 1) / bs), is_pd(wf->model) ? 3u : 1u), block(bs);
   // the grid minimum is the reference frequency of the models that have none set
   const bool own_grid = fgrid && (is_pd(wf->model) ? !(wf->fref > 0.0) : (wf->is_eccentric && !(wf->fref_ecc > 0.0)));
-  if (own_grid) {
-    const int eb = n_ev >= 16 ? 16 : (n_ev >= 4 ? 4 : 1);
+  const bool loop = own_grid && nf <= (is_pd(wf->model) ? GRID_MIN_LOOP_PD : GRID_MIN_LOOP_TF);
+  if (own_grid && !loop) {
+    // events per block: 64 lanes each where the grid has loads for them (4 a lane)
+    int eb = n_ev >= 16 ? 16 : (n_ev >= 4 ? 4 : 1);
+    while (n_ev >= 16 && eb < 256 && 1024 / eb > 8 && (1024 / eb) * 4 > nf) eb *= 2;
     hipLaunchKernelGGL(k_grid_min, dim3((unsigned)((n_ev + eb - 1) / eb)), dim3(1024), 0, st, fgrid, n_ev, nf, eb, rec);
   }
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid, rec);
+    hipLaunchKernelGGL(kern, grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid, loop ? fgrid : nullptr, nf, rec);
   };
   if (wf->model == GWF_MODEL_IMRPHENOMD)
     go(k_setup<GWF_MODEL_IMRPHENOMD, 4>);

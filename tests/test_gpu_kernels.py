@@ -265,6 +265,25 @@ def test_ragged_order_changes_no_result(n, longest):
     assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
 
 
+@pytest.mark.parametrize('n', [1, 17, 300])
+@pytest.mark.parametrize('nf', [1, 2, 12, 13, 24, 25, 80])
+def test_grid_minimum_on_short_grids(n, nf):
+    """The same on grids that the setup's lanes look through themselves and
+    just longer ones: IMRPhenomD, NRTidalv2 and eccentric TaylorF2 bit for bit
+    as with the reference frequency set to the minimum."""
+    from gwfast_amd.waveforms import IMRPhenomD, IMRPhenomD_NRTidalv2, TaylorF2_RestrictedPN
+    rng = np.random.default_rng(7)
+    f = rng.uniform(5., 60., (nf, n))
+    f[rng.integers(0, nf, n), np.arange(n)] = 4.5
+    if nf > 1:
+        f[(np.argmin(f, axis=0) + 1) % nf, np.arange(n)] = np.nan
+    for make, key, P in ((IMRPhenomD, 'fRef', 11), (IMRPhenomD_NRTidalv2, 'fRef', 13),
+                         (lambda **k: TaylorF2_RestrictedPN(is_eccentric=True, **k), 'fRef_ecc', 12)):
+        ev = _events(P, n, 5)
+        got, want = make().Phi(f, **ev), make(**{key: 4.5}).Phi(f, **ev)
+        assert np.array_equal(got, want, equal_nan=True) and np.isfinite(got[np.isfinite(f)]).all()
+
+
 # z and SiLU(z): past the exponential's overflow (-88.72) the quotient is -0, -inf / inf has no value
 SILU_EXTREMES = [(-3.0e38, -0.), (-1e30, -0.), (-1e10, -0.), (-1000., -0.), (-100., -0.), (0., 0.), (-0., -0.),
                  (80., 80.), (1000., 1000.), (1e30, 1e30), (3.0e38, 3.0e38), (np.inf, np.inf), (-np.inf, np.nan),
