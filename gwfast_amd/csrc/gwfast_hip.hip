@@ -205,8 +205,8 @@ constexpr int64_t GRID_MIN_LOOP_PD = 12, GRID_MIN_LOOP_TF = 24;
 
 template <int MODEL, int NT>
 __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const double* __restrict__ par, int64_t ld,
-                                               int64_t n_ev, bool own_grid, const double* __restrict__ fgrid,
-                                               int64_t nf, double* __restrict__ rec) {
+                                               int64_t n_ev, const double* __restrict__ fgrid, int64_t nf,
+                                               double* __restrict__ rec) {
   // IMRPhenomD models: NT lanes per event, lane tk evaluating tangent tk
   // (setup_waveform_split), and grid row y the phase's coefficients, the
   // amplitude's or (one lane per event) the event's constants: three chains of
@@ -234,11 +234,9 @@ __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const d
     }
   }
   double f0;
-  if (fgrid) {  // minimum of the caller's grid column (waveforms.py:1139)
-    f0 = fgrid[e];
+  if (fgrid) {  // minimum of the caller's grid column (waveforms.py:1139), nf = 0: from k_grid_min
+    f0 = nf > 0 ? fgrid[e] : r[REC_F0];
     for (int64_t i = 1; i < nf; ++i) f0 = fmin(f0, fgrid[i * n_ev + e]);
-  } else if (own_grid) {  // the same from k_grid_min
-    f0 = r[REC_F0];
   } else {  // first grid point: 10**log10(fmin) for geomspace, fmin for linspace
     f0 = net.lin ? net.fmin : grid_f(log10(net.fmin), log10(net.fmin), 0, 1);
   }
@@ -2901,7 +2899,7 @@ int launch_setup(const gwf_waveform* wf, const NetK& net, const double* par, int
     hipLaunchKernelGGL(k_grid_min, dim3((unsigned)((n_ev + eb - 1) / eb)), dim3(1024), 0, st, fgrid, n_ev, nf, eb, rec);
   }
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid, loop ? fgrid : nullptr, nf, rec);
+    hipLaunchKernelGGL(kern, grid, block, 0, st, *wf, net, par, ld, n_ev, own_grid ? fgrid : nullptr, loop ? nf : 0, rec);
   };
   if (wf->model == GWF_MODEL_IMRPHENOMD)
     go(k_setup<GWF_MODEL_IMRPHENOMD, 4>);

@@ -275,3 +275,37 @@ def test_screened_fisher_matches_plain_and_gains(trained):
     assert torch.equal(a['idx'], b['idx'])
     assert torch.equal(a['F'], b['F'])
     assert a['n_exact_snr'] < b['n_exact_snr']
+
+
+@pytest.mark.parametrize('B', [1, 63, 65, 1000, 4097])
+def test_output_layer_backward_and_column_sums(B):
+    """gwf_head_backward and gwf_colsum, the building blocks of a backward pass
+    that gwf_mlp_backward does in one, against 64-bit sums: dH a single FP32
+    product, sums of B terms within B roundings of 2^-24 of the sum of moduli
+    (the order of their partial sums is not fixed)."""
+    import torch
+    from gwfast_amd import _engine as E, _native as N
+    rng = np.random.default_rng(B)
+    dev = lambda a: torch.as_tensor(np.asarray(a, dtype=np.float32)).cuda()
+    H, w, g = dev(rng.normal(size=(B, 256))).to(torch.bfloat16), dev(rng.normal(size=256)), dev(rng.normal(size=B))
+    dH, dw, db = torch.empty((B, 256), device='cuda'), torch.empty(256, device='cuda'), torch.empty(1, device='cuda')
+    s = N.stream_ptr()
+    E.call('gwf_head_backward', N.ptr(H), N.ptr(w), N.ptr(g), B, N.ptr(dH), N.ptr(dw), N.ptr(db), s)
+    assert torch.equal(dH, g[:, None] * w[None, :])
+    f64 = lambda t: t.to(torch.float64).cpu().numpy()
+    h, g64 = f64(H), f64(g)
+
+    def close(t, ref, moduli):
+        assert np.all(np.abs(f64(t) - ref) <= (B + 1) * 2. ** -24 * moduli)
+
+    close(dw, g64 @ h, np.abs(g64) @ np.abs(h))
+    close(db, g64.sum(), np.abs(g64).sum())
+    X = dev(rng.normal(size=(B, 37)))
+    x, Xb = f64(X), X.to(torch.bfloat16)
+    xb = f64(Xb)
+    out = torch.ones(37, device='cuda')
+    for X32, X16, weight, acc in ((X, None, None, 0), (X, None, g, 1), (None, Xb, None, 1), (None, Xb, g, 0)):
+        start = f64(out) if acc else np.zeros(37)
+        a, v = xb if X32 is None else x, np.ones(B) if weight is None else g64
+        E.call('gwf_colsum', N.ptr(X32), N.ptr(X16), N.ptr(weight), B, 37, N.ptr(out), acc, s)
+        close(out, start + v @ a, np.abs(start) + np.abs(v) @ np.abs(a))
