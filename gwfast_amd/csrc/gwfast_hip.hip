@@ -1741,46 +1741,59 @@ __global__ __launch_bounds__(BLOCK) void k_vjp_pairs(const double* __restrict__ 
 }
 
 // VJP of the strain, bound by the read of J: a block per event, whose lanes
-// take a point and all P parameters at a time, P + 1 loads in flight (gh, read
-// across events, once instead of once per parameter, and shared with the
-// neighbouring blocks in the XCD's L2), sums added through LDS in wave order.
-// 500 events x 2000 points, P = 11: 66 -> 31 us, 6 TB/s; a wave per parameter
-// and event read gh eleven times, a line of it per lane.
-template <int P>
-__global__ __launch_bounds__(BLOCK) void k_vjp(const double* __restrict__ J, const double* __restrict__ gh,
-                                               int64_t n_ev, int64_t nf, double tc_scale, double* __restrict__ g) {
-  __shared__ double part[WAVES_PER_BLOCK][P];
+// take a point and all PB parameters of a pass at a time, PB + 1 loads in
+// flight (gh, read across events, once per pass instead of once per parameter,
+// and shared with the neighbouring blocks in the XCD's L2), sums added through
+// LDS in wave order.  500 events x 2000 points, P = 11: 66 -> 28 us, 6.7 TB/s;
+// a wave per parameter and event read gh eleven times, a line of it per lane.
+template <int PB>
+__device__ __forceinline__ void vjp_pass(const double* __restrict__ J, const double* __restrict__ gh, int p0,
+                                         int64_t n_ev, int64_t nf, int64_t e, double tc_scale, double* __restrict__ g,
+                                         double (*part)[16]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const double* Je = J + 2 * ((int64_t)p0 * n_ev + e) * nf;
   const int64_t js = 2 * n_ev * nf;
+  double acc[PB];
+#pragma unroll
+  for (int p = 0; p < PB; ++p) acc[p] = 0.0;
+  for (int64_t i = threadIdx.x; i < nf; i += BLOCK) {
+    const double gr = gh[2 * (i * n_ev + e)], gi = gh[2 * (i * n_ev + e) + 1];
+    double re[PB], im[PB];
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+      re[p] = Je[p * js + 2 * i];
+      im[p] = Je[p * js + 2 * i + 1];
+    }
+    if constexpr (PB > 4) __builtin_amdgcn_sched_barrier(0);  // every load before the first use
+#pragma unroll
+    for (int p = 0; p < PB; ++p) acc[p] += gr * re[p] + gi * im[p];
+  }
+  const WaveSums<PB> sums(acc, lane);  // PB <= 64: one per lane
+  const int k = WaveSums<PB>::index(lane, 0);
+  if (k < PB) part[wave][k] = sums.v[0];
+  __syncthreads();
+  if (threadIdx.x < PB) {
+    double s = part[0][threadIdx.x];
+    for (int w = 1; w < WAVES_PER_BLOCK; ++w) s += part[w][threadIdx.x];
+    const int p = p0 + threadIdx.x;
+    g[p * n_ev + e] = p == 7 ? s * tc_scale : s;
+  }
+  __syncthreads();
+}
+// PT > 0: all P = PT parameters in one pass (the models' 11 to 14)
+template <int PT>
+__global__ __launch_bounds__(BLOCK) void k_vjp(const double* __restrict__ J, const double* __restrict__ gh, int P,
+                                               int64_t n_ev, int64_t nf, double tc_scale, double* __restrict__ g) {
+  __shared__ double part[WAVES_PER_BLOCK][16];
   for (int64_t b = blockIdx.x; b < n_ev; b += gridDim.x) {
     const int64_t e = near_block(b, n_ev);
-    const double* Je = J + 2 * e * nf;
-    double acc[P];
-#pragma unroll
-    for (int p = 0; p < P; ++p) acc[p] = 0.0;
-    for (int64_t i = threadIdx.x; i < nf; i += BLOCK) {
-      const double gr = gh[2 * (i * n_ev + e)], gi = gh[2 * (i * n_ev + e) + 1];
-      double re[P], im[P];
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        re[p] = Je[p * js + 2 * i];
-        im[p] = Je[p * js + 2 * i + 1];
-      }
-      __builtin_amdgcn_sched_barrier(0);  // every load before the first use
-#pragma unroll
-      for (int p = 0; p < P; ++p) acc[p] += gr * re[p] + gi * im[p];
+    if constexpr (PT > 0) {
+      vjp_pass<PT>(J, gh, 0, n_ev, nf, e, tc_scale, g, part);
+    } else {
+      int p = 0;
+      for (; p + 4 <= P; p += 4) vjp_pass<4>(J, gh, p, n_ev, nf, e, tc_scale, g, part);
+      for (; p < P; ++p) vjp_pass<1>(J, gh, p, n_ev, nf, e, tc_scale, g, part);
     }
-    const WaveSums<P> sums(acc, lane);  // P <= 64: one per lane
-    const int k = WaveSums<P>::index(lane, 0);
-    if (k < P) part[wave][k] = sums.v[0];
-    __syncthreads();
-    if (threadIdx.x < P) {
-      double s = part[0][threadIdx.x];
-      for (int w = 1; w < WAVES_PER_BLOCK; ++w) s += part[w][threadIdx.x];
-      const int p = threadIdx.x;
-      g[p * n_ev + e] = p == 7 ? s * tc_scale : s;
-    }
-    __syncthreads();
   }
 }
 
@@ -3420,8 +3433,8 @@ int gwf_strain_components(const gwf_waveform* wf, const gwf_detector* det, int32
   return strain_impl(wf, det, arm, params, ld, n_ev, f, n_f, nullptr, nullptr, comp_out, workspace, ws_bytes, stream);
 }
 
-// A model's rows on a grid of at least this many points take a block per event,
-// shorter ones (whose points would not fill it) a wave per parameter and event.
+// Grids of at least this many points take a block per event, shorter ones
+// (whose points would not fill it) a wave per parameter and event.
 // Pairs and block at P = 11: 1000 x 64 points 6.8 and 8.2 us, 6 x 10^4 x 5 101
 // and 346, 2 x 10^4 x 100 192 and 118, 5000 x 128 46 and 32.
 constexpr int64_t VJP_BLOCK_POINTS = 96;
@@ -3433,10 +3446,10 @@ int gwf_strain_vjp(const double* J, const double* gh, int32_t P, int64_t n_ev, i
   if ((int64_t)P * n_ev > (int64_t)0x7fffffff / WAVES_PER_BLOCK) return fail(-EINVAL, "too many events for one call");
   hipStream_t st = (hipStream_t)stream;
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(n_ev, 1 << 20)), dim3(BLOCK), 0, st, J, gh, n_ev, n_f,
-                       tcoal_scale, g_out);
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(n_ev, 1 << 20)), dim3(BLOCK), 0, st, J, gh, (int)P, n_ev,
+                       n_f, tcoal_scale, g_out);
   };
-  if (P < 11 || P > 14 || n_f < VJP_BLOCK_POINTS) {
+  if (n_f < VJP_BLOCK_POINTS) {
     const int64_t waves = (int64_t)P * n_ev;
     hipLaunchKernelGGL(k_vjp_pairs, dim3((unsigned)((waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK)), dim3(BLOCK), 0,
                        st, J, gh, (int)P, n_ev, n_f, tcoal_scale, g_out);
@@ -3446,8 +3459,10 @@ int gwf_strain_vjp(const double* J, const double* gh, int32_t P, int64_t n_ev, i
     go(k_vjp<12>);
   } else if (P == 13) {
     go(k_vjp<13>);
-  } else {
+  } else if (P == 14) {
     go(k_vjp<14>);
+  } else {
+    go(k_vjp<0>);
   }
   return hip_check(hipGetLastError(), "gwf_strain_vjp launch");
 }
