@@ -210,55 +210,59 @@ __global__ __launch_bounds__(1024) void k_grid_min(const double* __restrict__ f,
   if (ty == 0 && e < n_ev) rec[e * (int64_t)REC_DOUBLES + REC_F0] = red[tx];
 }
 
-// Grids of up to this many points are looked through by the setup's lanes
-// themselves, the IMRPhenomD models' NT lanes per event and eccentric
-// TaylorF2's one: there a launch costs more than the loads (the whole waveform
-// call with k_grid_min and with the loop: 10^5 eccentric events x 1 point 120
-// and 95 us, one event x 9 points 16.9 and 14.6; one IMRPhenomD event x 8
-// points 25.8 and 22.1).
-constexpr int64_t GRID_MIN_LOOP_PD = 12, GRID_MIN_LOOP_TF = 24;
-
+// Grids of up to this many points are looked through by eccentric TaylorF2's
+// setup itself, one lane per event: there a launch costs more than the loads
+// (the whole waveform call with k_grid_min and with the loop: 10^5 events x 1
+// point 120 and 95 us, one event x 9 points 16.9 and 14.6; with the loop in
+// the IMRPhenomD models' setup too, every call of theirs took 0.6 us more).
+constexpr int64_t GRID_MIN_LOOP = 24;
+// Event constants of the IMRPhenomD models: one of an event's NT lanes up to
+// this many lanes, one lane per event above, where the chip is full (whole
+// setup, one of NT and one per event: NRTidalv2, 3000 events 25.4 and 27.0 us,
+// 10^4 55.2 and 48.1; IMRPhenomD, 3000 events 20.6 and 21.8, 10^4 35.0 and 31.2).
+constexpr int64_t SETUP_DENSE = 32768;
 template <int MODEL, int NT>
 __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const double* __restrict__ par, int64_t ld,
                                                int64_t n_ev, const double* __restrict__ fgrid, int64_t nf,
                                                double* __restrict__ rec) {
   // IMRPhenomD models: NT lanes per event, lane tk evaluating tangent tk
   // (setup_waveform_split), and grid row y the phase's coefficients, the
-  // amplitude's or (one lane per event) the event's constants: three chains of
-  // about the same length, which as one bound every batch that does not fill
-  // the chip (IMRPhenomD, one chain and three: 1 to 1000 events 32 and 19 us,
-  // 10^4 40 and 31, 3 x 10^4 81 and 78, 10^5 328 and 290; NRTidalv2 39 and 25,
-  // 48.7 and 48.1, 132 and 126, 449 and 406; the same split at every size, so
-  // that a record does not depend on the batch).  TaylorF2: one lane per event
+  // amplitude's or the event's constants: three chains of about the same
+  // length, which as one bound every batch that does not fill the chip
+  // (IMRPhenomD, one chain and three: 1 to 1000 events 32 and 19 us, 10^4 40
+  // and 31, 3 x 10^4 81 and 79, 10^5 328 and 286; NRTidalv2 39 and 24, 48.7 and
+  // 48.1, 132 and 126, 449 and 405; the same arithmetic at every size, so that
+  // a record does not depend on the batch).  TaylorF2: one lane per event
   constexpr int LPE = is_pd(MODEL) ? NT : 1;
   const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if constexpr (is_pd(MODEL)) {
-    if (blockIdx.y == 2) {  // the constants: one lane per event
-      if (tid < n_ev) setup_pd_consts<MODEL>(net, par, ld, tid, rec + tid * (int64_t)REC_DOUBLES);
-      return;
-    }
-  }
   const int64_t e = tid / LPE;
   const int tk = (int)(tid - e * LPE);
   if (e >= n_ev) return;
   double* r = rec + e * (int64_t)REC_DOUBLES;
-  if constexpr (is_pd(MODEL)) {
-    if (blockIdx.y == 1) {  // the amplitude, which has no reference frequency
-      setup_waveform_split<MODEL, PD_AMP>(w, par, ld, e, 1.0, r, tk);
-      return;
-    }
-  }
   double f0;
   if (fgrid) {  // minimum of the caller's grid column (waveforms.py:1139), nf = 0: from k_grid_min
-    f0 = nf > 0 ? fgrid[e] : r[REC_F0];
-    for (int64_t i = 1; i < nf; ++i) f0 = fmin(f0, fgrid[i * n_ev + e]);
+    if (is_pd(MODEL) || nf == 0) {
+      f0 = r[REC_F0];
+    } else {
+      f0 = fgrid[e];
+      for (int64_t i = 1; i < nf; ++i) f0 = fmin(f0, fgrid[i * n_ev + e]);
+    }
   } else {  // first grid point: 10**log10(fmin) for geomspace, fmin for linspace
     f0 = net.lin ? net.fmin : grid_f(log10(net.fmin), log10(net.fmin), 0, 1);
   }
-  if constexpr (is_pd(MODEL))
-    setup_waveform_split<MODEL, PD_PHASE>(w, par, ld, e, f0, r, tk);
-  else
+  if constexpr (is_pd(MODEL)) {
+    if (blockIdx.y == 0)
+      setup_waveform_split<MODEL, PD_PHASE>(w, par, ld, e, f0, r, tk);
+    else if (blockIdx.y == 1)
+      setup_waveform_split<MODEL, PD_AMP>(w, par, ld, e, f0, r, tk);
+    else {
+      const bool dense = n_ev * LPE > SETUP_DENSE;
+      const int64_t ec = dense ? tid : e;
+      if (dense ? tid < n_ev : tk == 0) setup_pd_consts<MODEL>(net, par, ld, ec, rec + ec * (int64_t)REC_DOUBLES);
+    }
+  } else {
     setup_event<MODEL, NT>(w, net, par, ld, e, f0, r);
+  }
 }
 
 // The records of gwf_snr_once (setup_event_snr), one lane per event: values of
@@ -2919,11 +2923,11 @@ int launch_setup(const gwf_waveform* wf, const NetK& net, const double* par, int
   const dim3 grid((unsigned)((nt + bs - 1) / bs), is_pd(wf->model) ? 3u : 1u), block(bs);
   // the grid minimum is the reference frequency of the models that have none set
   const bool own_grid = fgrid && (is_pd(wf->model) ? !(wf->fref > 0.0) : (wf->is_eccentric && !(wf->fref_ecc > 0.0)));
-  const bool loop = own_grid && nf <= (is_pd(wf->model) ? GRID_MIN_LOOP_PD : GRID_MIN_LOOP_TF);
+  const bool loop = own_grid && !is_pd(wf->model) && nf <= GRID_MIN_LOOP;
   if (own_grid && !loop) {
     // events per block: 64 lanes each where the grid has loads for them (4 a lane)
     int eb = n_ev >= 16 ? 16 : (n_ev >= 4 ? 4 : 1);
-    while (n_ev >= 16 && eb < 256 && 1024 / eb > 8 && (1024 / eb) * 4 > nf) eb *= 2;
+    while (eb < 128 && n_ev / eb > 512 && (1024 / eb) * 4 > nf) eb *= 2;
     hipLaunchKernelGGL(k_grid_min, dim3((unsigned)((n_ev + eb - 1) / eb)), dim3(1024), 0, st, fgrid, n_ev, nf, eb, rec);
   }
   auto go = [&](auto kern) {

@@ -493,3 +493,20 @@ def test_ragged_order_where_it_pays_and_where_not(n, kind):
     for e in (0, 1, 66, n - 1):
         one = S.fisher_device(sigs, wf, rows[:, e:e + 1].contiguous(), np.array([max(2, lengths[e])]))
         assert torch.equal(out[0][:, :, e], one[:, :, 0])
+
+
+@pytest.mark.parametrize('P,line', [(11, 32768 // 4), ('NRTidalv2', 32768 // 6)])
+def test_records_do_not_depend_on_the_batch(P, line):
+    """The setup's constants take one of an event's lanes or one lane per event
+    by the size of the batch: the same Fisher matrices bit for bit on both sides
+    of the line."""
+    import torch
+    from tests._common import NET_C1, hip_net
+    from gwfast_amd import signal as S
+    wf, n = _models()[P](), 5
+    rows = _model_rows(P, n, 8)
+    sigs = list(hip_net(wf, NET_C1, True).signals.values())
+    few = S.fisher_device(sigs, wf, rows, 70)
+    for m in (line - 1, line, line + 1, 2 * line):
+        many = S.fisher_device(sigs, wf, rows.repeat(1, m // n + 1)[:, :m].contiguous(), 70)
+        assert torch.equal(many, few.repeat(1, 1, m // n + 1)[:, :, :m])
