@@ -350,7 +350,7 @@ def catalogue_leg(net, n=100_000, res=1000, seed=21):
     nd = int(len(r['idxs_det']))
     return {'events_per_s': n / (t2 - t0), 'n_events': n, 'n_detected': nd, 'res': res,
             'device_chain_s': t1 - t0, 'files_s': t2 - t1, 'events_per_s_device_chain': n / (t1 - t0),
-            'path': 'forecast.compute_errs (gwf_snr, gwf_fisher on the detected events, gwf_check_fisher, '
+            'path': 'forecast.compute_errs (gwf_snr_once, gwf_fisher on the detected events, gwf_check_fisher, '
                     'gwf_cov_invert, gwf_sigma_sky_area) + forecast.to_file'}
 
 

@@ -5,7 +5,8 @@
 // (signal.py:658-777); the screen decides which events the exact SNR kernel
 // must still evaluate.
 //
-// Training building blocks (C ABI in include/gwfast_hip.h):
+// Training building blocks (C ABI in include/gwfast_hip.h; the package itself
+// trains with gwf_mlp_forward and gwf_mlp_backward, which do theirs in one):
 //   gwf_gemm_bf16      C = alpha op(A) op(B) + beta C on MFMA
 //                      (v_mfma_f32_16x16x16_bf16), fp32 accumulation, split-K
 //   gwf_bias_silu      Z = C + b, H = bf16(SiLU(Z))
@@ -16,6 +17,7 @@
 //   gwf_mse_grad       loss and dL/dy of the mean squared error
 //   gwf_adam           Adam on fp32 master weights + bf16 copies
 //   gwf_snr_features   event parameters -> standardised features
+// Training passes:
 //   gwf_mlp_forward    the whole network on standardised features, activations
 //                      kept for the backward pass
 //   gwf_mlp_backward   every gradient of sum(g y), from those activations
@@ -331,11 +333,11 @@ __global__ void k_features(const double* __restrict__ par, int64_t ld, int64_t n
 
 // ------------------------------------------------- fused training passes
 // Forward and backward of the whole network on a batch of B rows: at the
-// training sizes (256 to 8192 rows) the work is 2-7 GFLOP and a few MB, so
+// training sizes (256 to 8192 rows) the work is 0.2-7 GFLOP and a few MB, so
 // what bounds it is the number of launches and the serial chains in each.
-// As 31 launches of the kernels above 440 us per forward + backward of 4096
+// As 29 launches of the kernels above 438 us per forward + backward of 4096
 // rows (the column sums alone ten launches of 18-90 us each); as
-// k_mlp_fwd, k_mlp_bwd, k_mlp_dw and k_mlp_reduce 71 us (25, 19, 23 and 4).
+// k_mlp_fwd, k_mlp_bwd, k_mlp_dw and k_mlp_reduce 70 us (24, 19, 22 and 4).
 //
 // k_mlp_fwd / k_mlp_bwd: 16 rows per workgroup (4096 rows = 256 workgroups,
 // one per CU), wave w owns the 64 columns 64 w.. in four MFMA tiles; tile j

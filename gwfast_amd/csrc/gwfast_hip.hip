@@ -184,7 +184,7 @@ __device__ __forceinline__ int64_t near_event() {
 // neighbouring events (the columns' rows are then read in runs of eb doubles)
 // and 1024 / eb lanes per event, four loads in flight per lane.  As the
 // setup's own loop, one dependent load per point and event: 507 us of setup
-// at 500 events x 2000 points, with this kernel 30 + 5 us.
+// at 500 events x 2000 points, with this kernel 23 + 9 us.
 constexpr int REC_F0 = REC_SITE + (GWF_MAX_DETECTORS - 1) * SC_COUNT;
 __global__ __launch_bounds__(1024) void k_grid_min(const double* __restrict__ f, int64_t n_ev, int64_t nf, int eb,
                                                    double* __restrict__ rec) {
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void k_setup(gwf_waveform w, NetK net, const d
 
 // The records of gwf_snr_once (setup_event_snr), one lane per event: values of
 // the amplitude's slots alone, where k_setup's tangents and phase bound a large
-// batch (10^5 IMRPhenomD events: k_setup 310 us, this 81) and its chain a
+// batch (10^5 IMRPhenomD events: k_setup 286 us, this 81) and its chain a
 // small one (100 tidal TaylorF2 events 12 us, 7).
 template <int MODEL>
 __global__ __launch_bounds__(256) void k_setup_snr(gwf_waveform w, NetK net, const double* __restrict__ par, int64_t ld,
@@ -1250,7 +1250,7 @@ __global__ __launch_bounds__(128 * PC_EPB, 4 / PC_EPB) void k_fisher_pq(gwf_wave
 // longest event apart.  One block; clears the queue counters (counter[0],
 // counter[1]) and says in counter[2] whether there is an order.
 // What the order saves grows with the spread of the lengths (some 2 us per
-// chunk of it, once per batch); what it costs grows with n_ev: the sort 10 us
+// chunk of it, once per batch); what it costs grows with n_ev: the sort 30 us
 // at 2 x 10^4, and neighbouring events' results no longer written together.
 // Measured on IMRPhenomD events in five arms, as they come and ordered, the
 // spread in chunks against the line:
@@ -1587,7 +1587,7 @@ __global__ void k_fcut(gwf_waveform w, const double* __restrict__ par, int64_t l
 // per event, 2000 events leave most of the loads the chip can hold in flight
 // unused.  f and S are read across events, so a block's neighbours run on its
 // XCD (near_block), and a lane takes its neighbours' f by shuffles.  2000
-// events x 1000 points, P = 11: 141 -> 117 us, 3.0 TB/s (with four waves'
+// events x 1000 points, P = 11: 141 -> 115 us, 3.3 TB/s (with four waves'
 // sums by wave_sum 204 us, bound by the LDS of its shuffles).
 template <int P>
 __global__ __launch_bounds__(256) void k_gram(const double* __restrict__ J, const double* __restrict__ f,

@@ -210,7 +210,7 @@ int gwf_snr_prepared(const gwf_waveform* wf, const gwf_detector* dets, int32_t n
                      double* snrsq_out, const void* workspace, size_t ws_bytes, void* stream);
 /* gwf_fisher_prepared also keeps two queue counters after the records (the
  * network sum's producer / consumer launch), so its workspace is writable and
- * at least gwf_workspace_bytes(n_ev). */
+ * holds the records and those 256 bytes (gwf_workspace_bytes less the order). */
 int gwf_fisher_prepared(const gwf_waveform* wf, const gwf_detector* dets, int32_t n_det, int64_t n_ev, int32_t res,
                         int32_t arm, double* fisher_out, void* workspace, size_t ws_bytes, void* stream);
 
@@ -321,6 +321,9 @@ int gwf_check_fisher(const double* F, int32_t P, int64_t n_ev, double* evals_out
  * the network log SNR; events whose prediction falls inside a band around
  * the detection threshold are recomputed exactly.  bf16 arrays are passed
  * as void* (raw 16-bit patterns, round-to-nearest-even).
+ * The package trains with gwf_mlp_forward and gwf_mlp_backward; gwf_gemm_bf16,
+ * gwf_bias_silu, gwf_silu_backward, gwf_colsum, gwf_head_forward and
+ * gwf_head_backward are the same passes in parts, for callers of their own.
  * ---------------------------------------------------------------------- */
 
 /* C (M x N, row stride ldc, fp32) = alpha * sum_k A(m, k) B(k, n) + beta * C,
@@ -331,7 +334,8 @@ int gwf_gemm_bf16(int32_t M, int32_t N, int32_t K, float alpha, const void* A, i
                   const void* B, int64_t sbk, int64_t sbn, float beta, float* C, int64_t ldc, int32_t split_k,
                   void* stream);
 
-/* Z = C + bias (per column), H = bf16(SiLU(Z)); C, Z (M, N) fp32, Z_out may be NULL. */
+/* Z = C + bias (per column), H = bf16(SiLU(Z)); C, Z (M, N) fp32, Z_out may be NULL.
+ * SiLU(z) = z / (1 + exp(-z)): +inf at +inf, -0 below -88.8, NaN at -inf and NaN. */
 int gwf_bias_silu(const float* C, const float* bias, int64_t M, int32_t N, float* Z_out, void* H_out, void* stream);
 
 /* dZ = dH * SiLU'(Z) over n elements; either output may be NULL (not both). */
