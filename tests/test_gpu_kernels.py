@@ -510,3 +510,93 @@ def test_records_do_not_depend_on_the_batch(P, line):
     for m in (line - 1, line, line + 1, 2 * line):
         many = S.fisher_device(sigs, wf, rows.repeat(1, m // n + 1)[:, :m].contiguous(), 70)
         assert torch.equal(many, few.repeat(1, 1, m // n + 1)[:, :, :m])
+
+
+def test_captured_calls_follow_their_inputs():
+    """The SNR alone, a ragged batch (once with an order and once without, by
+    its lengths), strain rows with the grid's minimum and their VJP, recorded
+    into one HIP graph: every replay on new inputs in the same buffers, with
+    eager work between, gives the eager results bit for bit."""
+    import torch
+    from tests._common import NET_C1, hip_net
+    from gwfast_amd import _engine as E, _native as N, signal as S
+    wf, n, nf, res = _wf(11), 1200, 70, 130
+    sigs = list(hip_net(wf, NET_C1, True).signals.values())
+    dets, nd = S._dets(sigs), len(sigs)
+    det = sigs[1].c_struct()
+    nb = int(N.lib().gwf_workspace_bytes(n))
+    new = lambda *shape: torch.empty(shape, dtype=torch.float64, device='cuda')
+    wss = [torch.empty(nb, dtype=torch.uint8, device='cuda') for _ in range(3)]
+    rows, f, gh = new(11, n), new(nf, n), new(nf, n, 2)
+    lengths = torch.empty(n, dtype=torch.int32, device='cuda')
+    out = {'snr': new(5, n), 'F': new(11, 11, n), 'h': new(nf, n, 2), 'J': new(11, n, nf, 2), 'g': new(11, n)}
+
+    def calls():
+        s = N.stream_ptr()
+        E.call('gwf_snr_once', wf.c_struct(), dets, nd, N.ptr(rows), n, n, res, None, N.ptr(out['snr']), N.ptr(wss[0]), nb, s)
+        E.call('gwf_fisher_ragged', wf.c_struct(), dets, nd, N.ptr(rows), n, n, N.ptr(lengths), -1, N.ptr(out['F']),
+               N.ptr(wss[1]), nb, s)
+        E.call('gwf_strain', wf.c_struct(), S.ctypes_byref(det), 0, N.ptr(rows), n, n, N.ptr(f), nf, N.ptr(out['h']),
+               N.ptr(out['J']), N.ptr(wss[2]), nb, s)
+        E.call('gwf_strain_vjp', N.ptr(out['J']), N.ptr(gh), 11, n, nf, 86400.0, N.ptr(out['g']), s)
+
+    def fill(seed):
+        rng = np.random.default_rng(seed)
+        rows.copy_(E.to_dev(E.param_rows(_events(11, n, seed), False)))
+        f.copy_(E.to_dev(np.sort(rng.uniform(4., 40., (nf, n)), axis=0)))
+        gh.copy_(E.to_dev(rng.standard_normal((nf, n, 2))))
+        lengths.copy_(E.to_dev(rng.integers(2, 1500 if seed % 2 else 100, n).astype(np.int32), torch.int32))
+
+    fill(1)
+    calls()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        calls()
+    for seed in (2, 3, 4, 5):
+        fill(seed)
+        for o in out.values():
+            o.fill_(float('nan'))
+        graph.replay()
+        got = {k: o.clone() for k, o in out.items()}
+        calls()
+        torch.cuda.synchronize()
+        for k, o in out.items():
+            assert bool(torch.isfinite(o).all()) and torch.equal(got[k], o), (k, seed)
+
+
+@pytest.mark.parametrize('B', [300])
+def test_captured_training_step_follows_its_inputs(B):
+    """The training passes recorded into a HIP graph: every replay on new rows
+    gives the eager predictions and gradients bit for bit."""
+    import torch
+    from gwfast_amd import screen
+    sc = screen.SNRScreen(seed=4)
+    gen = torch.Generator(device='cuda').manual_seed(1)
+    X = torch.zeros((B, screen.KFEAT), dtype=torch.bfloat16, device='cuda')
+    g = torch.empty(B, dtype=torch.float32, device='cuda')
+    y, bt = sc.forward_train(X)
+
+    def calls():
+        sc.forward_train(X, bt)
+        sc.backward(X, bt, g)
+
+    def fill():
+        X[:, :screen.NFEAT].copy_(torch.randn((B, screen.NFEAT), device='cuda', generator=gen))
+        g.copy_(torch.randn(B, device='cuda', generator=gen))
+
+    fill()
+    calls()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        calls()
+    for _ in range(3):
+        fill()
+        y.fill_(float('nan'))
+        sc.grad.fill_(float('nan'))
+        graph.replay()
+        got = y.clone(), sc.grad.clone()
+        calls()
+        torch.cuda.synchronize()
+        assert bool(torch.isfinite(y).all()) and torch.equal(got[0], y) and torch.equal(got[1], sc.grad)
